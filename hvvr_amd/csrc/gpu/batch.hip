@@ -604,7 +604,7 @@ int hvvr_gpu_batch_autotune(hvvr_gpu_batch* b, hvvr_gpu_scene* s, const float* c
     if (rc)
         return rc;
     // coordinate descent over the shape's fields
-    const std::vector<uint32_t> largeC = {640, 1280, 2560}, hugeC = {256, 512, 1024}, giantC = {128, 256, 512},
+    const std::vector<uint32_t> largeC = {320, 640, 1280}, hugeC = {128, 256, 512}, giantC = {64, 128, 256},
                                 walkC = {256, 1024, 2048}, swizzleC = {0, 1}, streamsC = {1, 2, 4};
     struct Field {
         uint32_t LaunchShape::*member;

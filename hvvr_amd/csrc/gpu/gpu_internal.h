@@ -149,7 +149,7 @@ struct hvvr_gpu_view {
     hvvr::DeviceBuffer<hvvr::StackEntry> blockStacks;   // [blockCount][64]
     hvvr::DeviceBuffer<uint32_t> blockStackSize;        // [blockCount]
     hvvr::DeviceBuffer<uint32_t> recScratch;            // record node indices and emission order of the
-                                                        // queued tile-list configurations, per workgroup
+                                                        // colossal tile-list configuration, per workgroup
     hvvr::DeviceBuffer<uint32_t> tileLevel;             // [tileCount] tile-list configuration hint
     hvvr::DeviceBuffer<uint32_t> tileWork;              // [4][tileCount] per tile, last frame: BVH nodes
                                                         // tested by the tile traversal, its deepest stack,
@@ -173,7 +173,7 @@ struct hvvr_gpu_view {
                                                         // giant configurations and for the walk; [0], [2]
                                                         // and [4] are reduced from tileWork on request
     uint64_t listCapacity = 0;
-    uint32_t waveStackLimit = 64; // register stack entries per tile traversal (<= 64)
+    uint32_t waveStackLimit = 64; // block-stack entries a tile traversal starts from (<= 64)
     // foveated path (hvvr_gpu_view_set_foveated): cull planes and the t-max buffer apply to
     // foveated renders only
     bool foveated = false;
@@ -214,16 +214,18 @@ struct hvvr_gpu_view {
 namespace hvvr {
 
 // Per-frame scratch of the tile-list kernels taken from outside the view (the shared
-// scratch of hvvr_gpu_view_render_shared_scratch): the queued configurations' record
-// scratch, `groups[L]` persistent workgroups' worth for the large, huge, giant and
-// colossal configurations (L = 0..3), and the five tile queues, [5][tileCount].
+// scratch of hvvr_gpu_view_render_shared_scratch): the colossal configuration's record
+// scratch, the persistent workgroups of the large, huge, giant and colossal configurations
+// (groups[0..3]; the scratch holds groups[3] of them), and the five tile queues,
+// [5][tileCount].
 struct TileListScratch {
     uint32_t* rec;
     uint32_t* queues;
     uint32_t groups[4];
 };
-// the persistent workgroups of the large, huge, giant and colossal configurations whose
-// record scratch fits `words` 32-bit words (at most as many as a view's own scratch holds)
+// the persistent workgroups of the large, huge, giant and colossal configurations with
+// `words` 32-bit words of record scratch (the colossal one's; at most as many as a view's
+// own scratch holds)
 void tileListGroupsFor(size_t words, uint32_t groups[4]);
 
 // hvvr_gpu_view_create; with `deviceSetup` the sample hierarchy is allocated, not uploaded

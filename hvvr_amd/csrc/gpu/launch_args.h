@@ -38,6 +38,7 @@ struct BlockTraverseArgs {
 struct TileListArgs {
     const BVHNode* nodes;
     const FrustumPre* tilePre;
+    const FrustumPre* blockPre;
     const StackEntry* blockStacks;
     const uint32_t* blockStackSize;
     uint32_t* counts;
@@ -50,7 +51,7 @@ struct TileListArgs {
     uint32_t nextCounter;    // and of `nextQueue`
     unsigned long long* counters;
     uint32_t stackLimit;
-    uint32_t* recScratch; // per-workgroup record scratch of the queued configurations
+    uint32_t* recScratch; // per-workgroup record scratch of the colossal configuration
     // per tile, the queued configuration (1..4, 5 = the walk) whose capacity the tile's
     // last list on this scene needed; the queued kernels send a tile with a higher hint
     // straight to that queue (every configuration builds the same list, so a hint only
@@ -58,7 +59,8 @@ struct TileListArgs {
     uint32_t* tileLevel;
     uint32_t useHints; // 0 on a view's first frame of a scene
     uint32_t tileCount;
-    // per tile: [tile] BVH nodes tested, [tileCount + tile] deepest stack (plain stores:
+    // per tile: [tile] BVH nodes tested, [tileCount + tile] deepest stack (the block
+    // stack's entries where the list was ordered by sorting; plain stores:
     // one atomic per tile on a shared counter serialises every tile of the launch at one
     // memory channel)
     uint32_t* tileWork;
@@ -153,14 +155,15 @@ inline uint32_t remapUnits(const hvvr_gpu_view* v) { return ((v->width + 15) / 1
 // XCD x takes a contiguous run of tiles, which share BVH nodes and triangles in its L2).
 // None of these changes a result.
 struct LaunchShape {
-    uint32_t largeGroups = 2560, hugeGroups = 1024, giantGroups = 512, walkGroups = 1024;
+    uint32_t largeGroups = 1280, hugeGroups = 512, giantGroups = 256, walkGroups = 1024;
     uint32_t xcdSwizzle = 0;
     uint32_t streams = 1; // batches: chains the views are dealt to, each on its own stream
 };
-// the most persistent workgroups each queued configuration launches (its record scratch
-// is sized for them): as many as the chip holds at once; the colossal configuration, which
-// takes a CU's whole LDS and a few tiles of a dense scene, a quarter of the CUs
-enum : uint32_t { kMaxLargeGroups = 2560, kMaxHugeGroups = 1024, kMaxGiantGroups = 512, kMaxColossalGroups = 64 };
+// the most persistent workgroups each queued configuration launches: as many as the chip
+// holds at once (five of four waves, two of eight and one of sixteen per CU); the colossal
+// configuration, which takes a CU's whole LDS and the odd tile of a dense scene, a quarter
+// of the CUs (the record scratch is sized for it)
+enum : uint32_t { kMaxLargeGroups = 1280, kMaxHugeGroups = 512, kMaxGiantGroups = 256, kMaxColossalGroups = 64 };
 // 32-bit words of record scratch one view (or one batch chain) needs
 size_t tileListScratchWords();
 

@@ -12,7 +12,9 @@
 //                             tile's list at an offset claimed with one atomic add, so no
 //                             count pass and no scan are needed
 //   tileListQueueKernel<Cfg>  the same for the tiles a smaller configuration queued (large,
-//                             huge, giant, colossal: more records and deeper stacks)
+//                             huge, giant: more records, more waves per tile)
+//   tileSerialKernel          one wave64 per tile replaying the reference's walk over the
+//                             records, for the tiles those pass on
 //   tileWalkKernel            one wave64 per tile with a 4096-entry stack in LDS, for the
 //                             tiles no configuration holds (count pass, allocation, emit
 //                             pass)
@@ -219,136 +221,156 @@ __global__ __launch_bounds__(64) void blockTraverseBatchKernel(const BlockTraver
 }
 
 // ---------------------------------------------------------------------------------
-// Tile lists: traverseTiles (traverse_avx.h:412-527), one wave64 per tile.
+// Tile lists: traverseTiles (traverse_avx.h:412-527).
 //
 // The reference walks a tile's BVH cut depth-first from its block's sorted stack,
 // keeping the stack sorted by distance and emitting each visited node's surviving leaf
 // triangles in visit order. A node's test depends only on the tile frustum and the
-// node, not on when the walk reaches it, so the walk is split into three phases:
-//   A. tests: breadth-first over the nodes the walk will visit, 16 x Slots nodes per step
-//      (lane = node slot x child, each lane testing one child against every frustum
-//      axis; two node slots per lane group in the standard configuration, whose VGPRs
-//      bound its occupancy, four in the queued ones, whose LDS does). Each visited node
-//      becomes an LDS record: its final child mask (coarse test, refined when a leaf
-//      child passes), its leaf mask, the leaf mask of its stack entry and the index of
-//      its first internal child's record; the internal children that pass are appended
-//      as new records, in child order, with their distance keys.
-//   B. order: the reference's stack walk replayed over the records, with the stack in
-//      one VGPR pair: pops, the single-child shortcut, the sorted insertion (one ballot
-//      compares every entry), and the sequence of records whose leaves are emitted.
+// node, not on when the walk reaches it, so the work is split:
+//   A. tests: breadth-first over the nodes the walk will visit, 16 x Slots nodes per wave
+//      and step (lane = node slot x child, each lane testing one child against every
+//      frustum axis). Each visited node becomes an LDS record: its final child mask (coarse
+//      test, refined when a leaf child passes), its leaf mask, the leaf mask of its stack
+//      entry and the index of its first internal child's record; the internal children
+//      that pass are appended as new records, in child order.
+//   B. order: the emitting records (those with a passing leaf child) sorted into the walk's
+//      visit order.
 //   C. emit: the list length is summed, space is claimed with one atomic add, and the
 //      triangle ranges of the emitted leaves are written in order.
-// The dependent global loads per tile drop from one per visited node (~370 on the
-// 262k-triangle room scene) to one per 32 nodes.
 //
-// Phase B leaves out dead records, those with no passing child: the reference pops them
-// and does nothing else. Its stack stays sorted by key, ties newest on top (the block
-// stack arrives sorted and every insert lands at its sorted position), so a pop always
-// takes the least (key, newest) entry; an entry that changes nothing when popped can be
-// dropped without moving any other pop. The same holds for a record none of whose
-// subtree emits (a pass between phases A and B marks those dead too). A NaN key breaks
-// that order (it inserts on top of anything), and the register stack's empty lanes hold
-// -inf, so a tile with a NaN or infinite key, or with an unsorted block stack, goes to the
-// global-stack kernel, as does a tile whose records or stack exceed the capacity.
+// The visit order as a sort. The walk's stack is a priority queue: a pop takes the least
+// key, among equal keys the newest entry; a record whose node has exactly one passing
+// internal child hands over to it without a pop. A child's box lies inside its parent's, so
+// its distance key is never below its parent's, and the walk pops keys in ascending order.
+// With W the key at which a record is visited (its key; its parent's W for an only child):
+//   - records are visited in ascending W;
+//   - a record joins its parent's tree when their W are equal: it is then visited while
+//     that tree is (it is newer than anything else of that key), so a tree's records are
+//     consecutive, parents first, later children before earlier ones;
+//   - trees of equal W come newest first: in descending order of the visits of their
+//     roots' parents (rp: the parent record of the tree's root), children of one parent
+//     later ones first; block-stack entries are older than every pushed entry, among
+//     themselves the higher position first.
+// D numbers the records depth-first, later children first (the live ones: those with an
+// emitting record in their subtree). The order is then (W, W[rp] descending, D[rp]
+// descending, D): within one tree, and between trees under one parent, D decides; two
+// parents of equal W are visited in the order of their D when they lie in one tree or under
+// one parent, that is when their own rp agree. Where neighbours in the sorted order agree
+// in W and W[rp], but their parents' order is not decided that way, the tile's list is built
+// once more, its records ranked by a comparison that follows the rps up as far as it has to
+// (visitedBefore; two tiles of the 640x480 heightfield view, none of the room views, up to
+// one in twenty where boxes stand in a regular grid).
 //
-// Five configurations share the code. The standard one (680 records, a one-register
-// 64-entry stack, 8 KB of LDS) runs every tile; a tile it cannot hold is queued for
-// the large one (2048 records, a four-register 256-entry stack, 16 KB of LDS), what that
-// cannot hold for the huge one (4608 records, eight registers, 512 entries, 36 KB), and
-// so on to the giant one (10240 records, sixteen registers, 1024 entries, 80 KB) and the
-// colossal one (20480 records, the giant one's stack, all 160 KB of a CU's LDS); each
-// takes its queue with persistent workgroups, as many as fit the chip at once (the
-// colossal one with a few: it takes the odd tile of a dense scene seen through a wide
-// tile frustum, whose records, not its stack, outgrow the giant one; a 32-register stack
-// made its unrolled walk 20% slower). What none holds goes to the wave-per-tile walk with
-// its stack in LDS.
+// When the block's distance axis is not the tile's, the block-stack entries' keys are
+// measured along another axis than their descendants' and may exceed them. The subtree of
+// each entry (a family) is then ordered by itself first, with the entry's W = -inf (the
+// relative order of a family's visits does not depend on the other families), and a
+// second sort merges the families: with K the entry's key and E = max(K, W), records are
+// visited in ascending E; of equal E, first the trees pushed as such (W > K), newest first
+// (E[rp] descending; two families' that tie there are ranked as above), then the entries
+// of that key, the higher position first, each followed by what it uncovers (W <= K), in
+// its family's order.
+//
+// A NaN or infinite key has no place in this order, nor has an unsorted block stack: such
+// an irregular tile goes to the serial walk, as does one whose records exceed every
+// capacity.
+//
+// Replaying the walk over the records with a stack in registers, one wave per tile, took a
+// serial chain of some 500-850 cycles per record (84k of a 1080x1200 room eye's 170k cycles
+// per tile, 1.3M of 1.7M on a 2M-triangle scene); the sort has no such chain and takes any
+// number of waves.
+//
+// Four configurations share the code: the standard one takes every tile with one wave; a
+// tile it cannot hold is queued for the large one (four waves), what that cannot hold for
+// the huge one (eight waves), and so on to the giant one (sixteen waves, a CU's whole LDS),
+// each with as many persistent workgroups as fit the chip at once. Beyond it the colossal
+// configuration replays the walk with one wave (tileSerialBody), and what that cannot hold
+// goes to the wave-per-tile walk with its stack in LDS.
 // ---------------------------------------------------------------------------------
 // Record meta: first child record (bits 0..19), child mask (20..23), leaf mask (24..27),
 // stack-entry leaf mask (28..31).
 __device__ inline uint32_t metaMask(uint32_t m) { return (m >> 20) & 0xfu; }
 __device__ inline uint32_t metaLeaf(uint32_t m) { return (m >> 24) & 0xfu; }
 __device__ inline uint32_t metaEntry(uint32_t m) { return m >> 28; }
+__device__ inline uint32_t metaFirst(uint32_t m) { return m & 0xfffffu; }
 __device__ inline uint32_t packMeta(uint32_t first, uint32_t mask, uint32_t leaf, uint32_t entry) {
     return first | (mask << 20) | (leaf << 24) | (entry << 28);
 }
+// the passing internal children, whose records the walk follows (not those of an entry
+// with a leaf mask), and the passing leaf children
+__device__ inline uint32_t metaInner(uint32_t m) { return metaEntry(m) == 0u ? metaMask(m) & ~metaLeaf(m) : 0u; }
+__device__ inline uint32_t metaEmits(uint32_t m) { return metaMask(m) & metaLeaf(m); }
 
-// The standard configuration keeps the record index in bits 10..19 of a stack entry's
-// meta (records < 1024), so a pop needs no LDS read; the others stack record indices.
-// The standard configuration keeps every record array in LDS. The others keep only the
-// keys and metas the stack walk reads there; each record's node index and the emission
-// order go to a per-workgroup region of global scratch (their persistent workgroups
-// reuse it tile after tile), which halves their LDS and doubles the workgroups a CU holds
-// (the walk is latency-bound: throughput follows the resident waves).
+// 16 bytes of LDS per record: 680 records of one wave let a CU hold 14 tiles; 2016 records
+// five workgroups (20 waves), 4608 two (16 waves), 9984 one (16 waves).
 struct TileListSmall {
-    enum : uint32_t { RecCap = 680, StackCap = REG_STACK_CAP, Packed = 1, LdsRecords = 1, Level = 0, Slots = 2 };
-    using Stack = RegStack;
+    enum : uint32_t { RecCap = 680, Waves = 1, Slots = 2, Level = 0 };
 };
 struct TileListLarge {
-    enum : uint32_t { RecCap = 2048, StackCap = REG_STACK4_CAP, Packed = 0, LdsRecords = 0, Level = 1, Slots = 4 };
-    using Stack = RegStack4;
+    enum : uint32_t { RecCap = 2016, Waves = 4, Slots = 2, Level = 1, Occupancy = 5 };
 };
 struct TileListHuge {
-    enum : uint32_t { RecCap = 4608, StackCap = REG_STACK8_CAP, Packed = 0, LdsRecords = 0, Level = 2, Slots = 4 };
-    using Stack = RegStack8;
+    enum : uint32_t { RecCap = 4608, Waves = 8, Slots = 2, Level = 2, Occupancy = 4 };
 };
 struct TileListGiant {
-    enum : uint32_t { RecCap = 10240, StackCap = REG_STACK16_CAP, Packed = 0, LdsRecords = 0, Level = 3, Slots = 4 };
-    using Stack = RegStack16;
+    enum : uint32_t { RecCap = 9984, Waves = 16, Slots = 2, Level = 3, Occupancy = 4 };
 };
+// the serial walk's: keys and metas in LDS (all 160 KB), node indices and emission order in
+// global scratch, a sixteen-register stack
 struct TileListColossal {
-    enum : uint32_t { RecCap = 20480, StackCap = REG_STACK16_CAP, Packed = 0, LdsRecords = 0, Level = 4, Slots = 4 };
+    enum : uint32_t { RecCap = 20480, StackCap = REG_STACK16_CAP, Level = 4, Slots = 4 };
     using Stack = RegStack16;
 };
 
-// 32-bit words of one workgroup's scratch region: node indices, then 16-bit order entries
-template <class Cfg>
+// 32-bit words of one colossal workgroup's scratch region: node indices, then 16-bit order
+// entries
 constexpr uint32_t recScratchWords() {
-    return Cfg::LdsRecords ? 0u : ((Cfg::RecCap + Cfg::RecCap / 2 + 63u) & ~63u);
+    return (TileListColossal::RecCap + TileListColossal::RecCap / 2 + 63u) & ~63u;
 }
 
-// (the standard configuration keeps its emission order in bits 10..19 of recMeta, which
-// its stored metas leave free: entry i of the order in recMeta[i])
-template <class Cfg, bool InLds = bool(Cfg::LdsRecords)>
-struct TileListLdsRecords {
-    uint32_t recNode[Cfg::RecCap];
-};
-template <class Cfg>
-struct TileListLdsRecords<Cfg, false> {};
-
-template <class Cfg>
-struct TileListLds : TileListLdsRecords<Cfg> {
-    uint32_t recKey[Cfg::RecCap];  // float bits of the record's distance key; in phase C, the
-                                   // list length of emitted record i
-    uint32_t recMeta[Cfg::RecCap]; // packMeta(first child record, child mask, leaf mask,
-                                   // stack-entry leaf mask)
+enum : uint32_t {
+    kMaxTileChunks = 64,   // chunks of the records' up and down passes
+    kNoRecord = 0xffffu,   // the rp of a block-stack entry's tree
+    kOldest = 0xffffffffu, // ~W[rp] of such a tree: older than any pushed entry
+    kUncovered = 0xffffffc0u // merged families: the entries' own place, by position below it
 };
 
+// An emitting record as a sort element: W and ~W[rp] as order-preserving integers, D[rp]
+// (descending) << 16 | D, and rp[rp] << 16 | record.
 template <class Cfg>
-__device__ inline uint32_t metaFirst(uint32_t m) {
-    return Cfg::Packed ? (m & 0x3ffu) : (m & 0xfffffu);
-}
-// stack entry of record r with meta m, and back
-template <class Cfg>
-__device__ inline uint32_t stackEntry(uint32_t r, uint32_t m) {
-    return Cfg::Packed ? ((m & ~(0x3ffu << 10)) | (r << 10)) : r;
-}
-template <class Cfg>
-__device__ inline void fromStackEntry(uint32_t e, const TileListLds<Cfg>& sh, uint32_t& rec, uint32_t& meta) {
-    if (Cfg::Packed) {
-        rec = (e >> 10) & 0x3ffu;
-        meta = e;
-    } else {
-        rec = e;
-        meta = uniform(sh.recMeta[e]);
-    }
+struct TileListLds {
+    enum : uint32_t { ElemCap = Cfg::RecCap / 2 };
+    uint32_t meta[Cfg::RecCap]; // packMeta; after the passes, low bits: the emitting records' list
+    uint32_t node[Cfg::RecCap];
+    union {
+        struct {
+            uint32_t key[Cfg::RecCap]; // float bits of W
+            uint32_t aux[Cfg::RecCap]; // rp << 16 | live records in the subtree, then D
+        };
+        uint4 elem[ElemCap];
+    };
+    uint32_t appended[3]; // children appended in a step (several waves), in turn
+    uint32_t bad;         // a NaN or infinite key; later, an order the sort does not decide
+    uint32_t emitters;
+    uint32_t waveTotals[Cfg::Waves];
+    uint32_t listStart[2]; // 64-bit list start, and whether the list fits
+    uint32_t listFits;
+    uint16_t chunk[kMaxTileChunks + 1]; // first record of each chunk
+    uint16_t familyD[64];               // first D of each block-stack entry's family
+};
+
+// every wave's LDS accesses before it are complete and seen by the others after it
+template <uint32_t Waves>
+__device__ inline void tileSync() {
+    if constexpr (Waves == 1)
+        waveLdsSync();
+    else
+        __syncthreads();
 }
 
+// order-preserving integer of a float without NaN (both zeros alike)
+__device__ inline uint32_t orderedKey(float f) { return floatFlip(fbits(f + 0.0f)); }
 
-__device__ inline void stackInit(RegStack& st, float t, uint32_t m, uint32_t size, uint32_t lane) {
-    st.t = lane < size ? t : -INFINITY;
-    st.m = m;
-    st.size = size;
-}
 // One child box of a node, as one lane of a 4-lane node group loads it.
 struct ChildBox {
     float b0, b1, b2, b3, b4, b5; // bounds[k][child]
@@ -373,12 +395,702 @@ __device__ inline ChildBox loadChildBox(const BVHNode* __restrict__ nodes, uint3
     return x;
 }
 
+// A tile's frustum as constant memory (written by an earlier kernel): its ~100 coefficients
+// come by scalar loads. The pointer is opaque, so each step loads them where it tests its
+// boxes (scalar cache hits): hoisted out of the loop they spill.
+__device__ inline const FrustumPre* stepFrustum(const FrustumPre* f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using ConstF = const __attribute__((address_space(4))) FrustumPre;
+    ConstF* p = (ConstF*)f;
+    asm volatile("" : "+s"(p));
+    return (const FrustumPre*)p;
+#else
+    return f;
+#endif
+}
+
+// The tests of S nodes per lane group: pass[k] = whether this lane's child of slot k
+// passes. Every lane active; wave-uniform `f`. (`&` rather than `&&` throughout: no branch
+// per lane condition.)
+template <uint32_t S>
+__device__ inline void testChildBoxes(const FrustumPre* __restrict__ f, const ChildBox (&X)[S], const bool (&valid)[S],
+                                      uint32_t lane, bool (&pass)[S]) {
+    const uint32_t s = lane >> 2;
+    bool refine[S];
+    uint64_t need[S];
+    uint32_t nNeed = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < S; k++) {
+        pass[k] = valid[k] & childCoarsePass(f, X[k].b0, X[k].b1, X[k].b2, X[k].b3, X[k].b4, X[k].b5);
+        const uint32_t m = uint32_t(ballot(pass[k]) >> (4 * s)) & 0xfu;
+        // refine only nodes with a passing leaf child (traverse_avx.h:447-452)
+        refine[k] = pass[k] & ((m & X[k].leafMask) != 0u);
+        need[k] = ballot(refine[k]);
+        nNeed += uint32_t(__builtin_popcountll(need[k]));
+    }
+    if (nNeed == 0u)
+        return;
+    if (nNeed < 64u) {
+        // Few boxes need the 12-axis test (typically a sixth of the lanes): move them to
+        // lanes 0 .. nNeed - 1 with forward permutes (every other lane sends to lane 63,
+        // which then holds no needed box), test them in one pass, and read each verdict
+        // back from the ballot.
+        uint32_t d[S];
+        float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f, g3 = 0.0f, g4 = 0.0f, g5 = 0.0f;
+        uint32_t base = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < S; k++) {
+            const uint32_t nk = uint32_t(__builtin_popcountll(need[k]));
+            d[k] = refine[k] ? base + lanesBelow(need[k]) : 63u;
+            const bool mine = lane >= base && lane < base + nk; // slot k's boxes land here
+            auto take = [&](float& gq, float v) {
+                const uint32_t x = uint32_t(__builtin_amdgcn_ds_permute(int(d[k] << 2), int(fbits(v))));
+                gq = mine ? bitsf(x) : gq;
+            };
+            take(g0, X[k].b0);
+            take(g1, X[k].b1);
+            take(g2, X[k].b2);
+            take(g3, X[k].b3);
+            take(g4, X[k].b4);
+            take(g5, X[k].b5);
+            base += nk;
+        }
+        const bool cull = childRefineCull(f, g0, g1, g2, g3, g4, g5);
+        const uint64_t culled = ballot(cull & (lane < nNeed));
+#pragma unroll
+        for (uint32_t k = 0; k < S; k++)
+            pass[k] &= !(refine[k] & (((culled >> d[k]) & 1ull) != 0ull));
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < S; k++) {
+            const bool cullK = childRefineCull(f, X[k].b0, X[k].b1, X[k].b2, X[k].b3, X[k].b4, X[k].b5);
+            pass[k] &= !(refine[k] & cullK);
+        }
+    }
+}
+
+// What the lists' space and statistics of a finished tile take from its first thread:
+// claims `total` entries; returns the start (and whether the list fits) to every lane of
+// the calling wave.
+__device__ inline uint64_t claimList(const TileListArgs& g, uint32_t tile, uint32_t total, uint32_t visits,
+                                     uint32_t deepest, uint32_t lane, bool& fits) {
+    unsigned long long start = 0;
+    if (lane == 0)
+        start = atomicAdd(&g.counters[3], (unsigned long long)total);
+    start = (uint64_t(readLane(uint32_t(start >> 32), 0)) << 32) | readLane(uint32_t(start), 0);
+    fits = start + total <= g.capacity;
+    if (lane == 0) {
+        g.counts[tile] = total;
+        g.offsets[tile] = uint32_t(start);
+        if (!fits)
+            atomicOr(&g.counters[1], 1ull);
+        g.tileWork[tile] = visits;
+        g.tileWork[g.tileCount + tile] = deepest;
+    }
+    return start;
+}
+
+// the smallest queued configuration that holds a tile of `records`, for its next frame
+__device__ inline uint32_t levelFor(uint32_t records) {
+    return records <= TileListLarge::RecCap ? 1u : records <= TileListHuge::RecCap ? 2u
+                                               : records <= TileListGiant::RecCap  ? 3u
+                                                                                   : 4u;
+}
+
+// x before y in the visit order (the first three words)
+__device__ inline bool elemLess(const uint4& x, const uint4& y) {
+    return x.x < y.x || (x.x == y.x && (x.y < y.y || (x.y == y.y && x.z < y.z)));
+}
+
+// Sorts sh.elem[0, n) ascending (a bitonic network whose comparators all point up, so the
+// missing elements past n need no padding). Comparator i of a stage of stride up to 64
+// touches the aligned 128 elements of its 64-comparator block, which one wave holds: such
+// stages need no workgroup barrier.
+template <class Cfg>
+__device__ inline void sortElements(TileListLds<Cfg>& sh, uint32_t n, uint32_t tid) {
+    constexpr uint32_t T = 64 * Cfg::Waves;
+    uint32_t P = 2;
+    while (P < n)
+        P <<= 1;
+    auto exchange = [&](uint32_t lo, uint32_t hi) {
+        if (hi < n) {
+            const uint4 a = sh.elem[lo], b = sh.elem[hi];
+            if (elemLess(b, a)) {
+                sh.elem[lo] = b;
+                sh.elem[hi] = a;
+            }
+        }
+    };
+    tileSync<Cfg::Waves>();
+    for (uint32_t size = 2; size <= P; size <<= 1) {
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            if (Cfg::Waves > 1 && stride > 64u)
+                __syncthreads();
+            const bool flip = stride == size >> 1;
+#pragma unroll 1
+            for (uint32_t i = tid; i < P / 2; i += T) {
+                const uint32_t off = i & (stride - 1u), base = (i - off) << 1;
+                exchange(base + off, flip ? base + size - 1u - off : base + off + stride);
+            }
+            if (Cfg::Waves > 1 && stride > 64u)
+                __syncthreads();
+            else
+                waveLdsSync();
+        }
+    }
+    tileSync<Cfg::Waves>();
+}
+
+enum class TileResult : uint32_t { Done, TooBig, Irregular, Undecided };
+
+// The block-stack entry whose family holds the record numbered d: the least position whose
+// family begins at or before it (the D go up as the positions go down, and an empty family
+// begins where the next one does).
+template <class Cfg>
+__device__ inline uint32_t familyOf(const TileListLds<Cfg>& sh, uint32_t n0, uint32_t d) {
+    uint32_t lo = 0, hi = n0 - 1u;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (sh.familyD[mid] <= d)
+            hi = mid;
+        else
+            lo = mid + 1u;
+    }
+    return lo;
+}
+
+// Whether the walk visits record x before y, from the records' W, D and rp, whatever ties:
+// the order stated above, with "newest first" followed to the parents as often as needed
+// (each turn replaces both records by parents, so it ends). `families`: W is relative to the
+// record's block-stack entry, whose key is in `bs`.
+template <class Cfg>
+__device__ bool visitedBefore(const TileListLds<Cfg>& sh, uint32_t x, uint32_t y, bool families, uint32_t n0,
+                              const StackEntry* bs) {
+    for (;;) {
+        const uint32_t ax = sh.aux[x], ay = sh.aux[y];
+        const uint32_t wx = orderedKey(bitsf(sh.key[x])), wy = orderedKey(bitsf(sh.key[y]));
+        uint32_t fx = 0, fy = 0;
+        if (families) {
+            fx = familyOf(sh, n0, ax & 0xffffu);
+            fy = familyOf(sh, n0, ay & 0xffffu);
+        }
+        if (fx == fy) {
+            if (wx != wy)
+                return wx < wy;
+            if ((ax >> 16) == (ay >> 16))
+                return (ax & 0xffffu) < (ay & 0xffffu);
+            if ((ax >> 16) == kNoRecord)
+                return false;
+            if ((ay >> 16) == kNoRecord)
+                return true;
+        } else {
+            const uint32_t kx = orderedKey(bs[fx].tMin), ky = orderedKey(bs[fy].tMin);
+            const uint32_t ex = wx > kx ? wx : kx, ey = wy > ky ? wy : ky;
+            if (ex != ey)
+                return ex < ey;
+            if (!(wx > kx) || !(wy > ky))
+                return (wx > kx) || (!(wy > ky) && fx > fy);
+        }
+        x = ay >> 16; // the one whose tree was pushed later comes first
+        y = ax >> 16;
+    }
+}
+
+// Builds one tile's list with the workgroup's Cfg::Waves waves (thread `tid`). `rank`: by
+// comparing every two emitting records (visitedBefore) instead of sorting.
+template <class Cfg>
+__device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t tile, uint32_t tid,
+                                   bool rank) {
+    constexpr uint32_t Waves = Cfg::Waves, T = 64 * Waves, RecCap = Cfg::RecCap;
+    constexpr uint32_t ElemCap = TileListLds<Cfg>::ElemCap;
+    const uint32_t lane = tid & 63u, wave = Waves == 1 ? 0u : uniform(tid >> 6);
+    const BVHNode* __restrict__ nodes = g.nodes;
+    const uint32_t block = tile / TILES_PER_BLOCK;
+    const FrustumPre* __restrict__ f = g.tilePre + tile;
+    const uint32_t n0 = g.blockStackSize[block];
+    if (n0 == 0 || f->degenerate) {
+        if (tid == 0) {
+            g.counts[tile] = 0u;
+            g.offsets[tile] = 0u;
+            g.tileWork[tile] = 0u;
+            g.tileWork[g.tileCount + tile] = 0u;
+        }
+        return TileResult::Done;
+    }
+    auto give = [&](TileResult r) {
+        if (tid == 0) {
+            g.counts[tile] = 0u;
+            g.offsets[tile] = 0u;
+        }
+        return r;
+    };
+    if (n0 > g.stackLimit)
+        return give(TileResult::TooBig);
+
+    // ---- phase A: node tests, breadth-first ----
+    const StackEntry* bs = g.blockStacks + size_t(block) * BLOCK_STACK_SIZE;
+    const uint32_t axis = uint32_t(f->distanceAxis);
+    const bool families = g.blockPre[block].distanceAxis != f->distanceAxis;
+    bool bad = false;
+    if (wave == 0) {
+        const float t = lane < n0 ? bs[lane].tMin : 0.0f;
+        if (lane < n0) {
+            const uint32_t m = bs[lane].nodeMask;
+            sh.node[lane] = m & STACK_NODE_MASK;
+            sh.key[lane] = fbits(families ? -INFINITY : t);
+            sh.meta[lane] = packMeta(0u, 0u, 0u, m >> 28);
+            sh.aux[lane] = kNoRecord << 16;
+        }
+        const float above = __shfl_down(t, 1);
+        bad = !(fabsf(t) <= FLT_MAX) || (lane + 1u < n0 && t < above);
+        if (lane == 0) {
+            sh.bad = 0u;
+            sh.emitters = 0u;
+            sh.appended[0] = 0u;
+        }
+    }
+    tileSync<Waves>();
+    uint32_t nrec = n0, chunks = 0, chunkEnd = 0;
+    {
+        constexpr uint32_t S = Cfg::Slots; // records per lane group and step
+        const uint32_t s = lane >> 2, c = lane & 3u;
+        const uint64_t groupBelow = (1ull << (4 * s)) - 1ull;
+        uint32_t turn = 0;
+        for (uint32_t head = 0; head < nrec;) {
+            // this step tests records [head, end), S per lane group (so their node loads
+            // overlap); the children it appends start at nrec
+            const uint32_t end = head + 16 * S * Waves < nrec ? head + 16 * S * Waves : nrec;
+            // a chunk: up to T records whose children all lie past it
+            if (end > chunkEnd) {
+                if (chunks == kMaxTileChunks)
+                    return give(TileResult::TooBig);
+                if (tid == 0)
+                    sh.chunk[chunks] = uint16_t(head);
+                chunks++;
+                chunkEnd = head + T < nrec ? head + T : nrec;
+            }
+            uint32_t recI[S], nodeR[S], entryR[S], rpR[S];
+            float wR[S];
+            bool valid[S], pass[S];
+#pragma unroll
+            for (uint32_t k = 0; k < S; k++) {
+                recI[k] = head + 16 * (k * Waves + wave) + s;
+                valid[k] = recI[k] < end;
+                nodeR[k] = entryR[k] = rpR[k] = 0;
+                wR[k] = 0.0f;
+                if (valid[k]) {
+                    nodeR[k] = sh.node[recI[k]];
+                    entryR[k] = metaEntry(sh.meta[recI[k]]);
+                    wR[k] = bitsf(sh.key[recI[k]]);
+                    rpR[k] = sh.aux[recI[k]] >> 16;
+                }
+            }
+            ChildBox X[S];
+#pragma unroll
+            for (uint32_t k = 0; k < S; k++)
+                X[k] = ChildBox{};
+            if (Waves == 1 || head + 16 * wave < end) { // (a wave without a record waits)
+#pragma unroll
+                for (uint32_t k = 0; k < S; k++)
+                    X[k] = loadChildBox(nodes, nodeR[k], c, axis);
+                testChildBoxes<S>(stepFrustum(f), X, valid, lane, pass);
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < S; k++)
+                    pass[k] = false;
+            }
+            // internal children are pushed only from entries without a leaf mask
+            // (traverse_avx.h:476-483)
+            bool inner[S];
+            uint64_t bi[S];
+            uint32_t total = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < S; k++) {
+                inner[k] = pass[k] && ((X[k].leafMask >> c) & 1u) == 0u && entryR[k] == 0u;
+                bi[k] = ballot(inner[k]);
+                total += uint32_t(__builtin_popcountll(bi[k]));
+            }
+            uint32_t base = nrec;
+            if constexpr (Waves > 1) {
+                uint32_t at = 0;
+                if (lane == 0)
+                    at = atomicAdd(&sh.appended[turn], total);
+                base += readLane(at, 0);
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < S; k++) {
+                const uint32_t maskK = uint32_t(ballot(pass[k]) >> (4 * s)) & 0xfu;
+                const uint32_t slot = base + lanesBelow(bi[k]);
+                const bool only = __builtin_popcount(uint32_t(bi[k] >> (4 * s)) & 0xfu) == 1;
+                if (inner[k] && slot < RecCap) {
+                    const float w = only ? wR[k] : X[k].key;
+                    sh.node[slot] = nodeR[k] + X[k].childOffset;
+                    sh.key[slot] = fbits(w);
+                    sh.meta[slot] = 0u;
+                    sh.aux[slot] = (w == wR[k] ? rpR[k] : recI[k]) << 16;
+                }
+                if (valid[k] && c == 0) {
+                    const uint32_t first = base + uint32_t(__builtin_popcountll(bi[k] & groupBelow));
+                    sh.meta[recI[k]] = packMeta(first, maskK, X[k].leafMask, entryR[k]);
+                }
+                base += uint32_t(__builtin_popcountll(bi[k]));
+                // (a key below its parent's W has no place in the order; boxes that nest
+                // have none)
+                bad |= inner[k] && (!(fabsf(X[k].key) <= FLT_MAX) || X[k].key < wR[k]);
+            }
+            head = end;
+            if constexpr (Waves > 1) {
+                // the next step's counter: last used two steps ago, read before the last
+                // barrier
+                const uint32_t next = turn == 2u ? 0u : turn + 1u;
+                if (tid == 0)
+                    sh.appended[next] = 0u;
+                __syncthreads();
+                nrec += uniform(sh.appended[turn]);
+                turn = next;
+            } else {
+                nrec = base;
+                waveLdsSync();
+            }
+            if (nrec > RecCap)
+                return give(TileResult::TooBig);
+        }
+    }
+    if (ballot(bad) != 0ull && lane == 0)
+        sh.bad = 1u;
+    if (tid == 0)
+        sh.chunk[chunks] = uint16_t(nrec);
+    tileSync<Waves>();
+    if (uniform(sh.bad) != 0u)
+        return give(TileResult::Irregular);
+
+    // ---- phase B: the emitting records in visit order ----
+    // Up: the live records of each subtree (children lie in later chunks than their parent).
+#pragma unroll 1
+    for (uint32_t k = chunks; k-- > 0;) {
+        const uint32_t r = sh.chunk[k] + tid;
+        if (r < sh.chunk[k + 1]) {
+            const uint32_t m = sh.meta[r], first = metaFirst(m);
+            const uint32_t n = uint32_t(__builtin_popcount(metaInner(m)));
+            uint32_t live = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (j < n)
+                    live += sh.aux[first + j] & 0xffffu;
+            if (live != 0u || metaEmits(m) != 0u)
+                sh.aux[r] |= live + 1u;
+        }
+        tileSync<Waves>();
+    }
+    // Down: D, from the block-stack entries, the highest position first.
+    if (wave == 0) {
+        const uint32_t q = n0 - 1u - lane;
+        const uint32_t a = lane < n0 ? sh.aux[q] : 0u, live = a & 0xffffu;
+        const uint32_t d = 1u + waveInclusiveScan(live) - live;
+        if (lane < n0) {
+            sh.aux[q] = (a & 0xffff0000u) | d;
+            sh.familyD[q] = uint16_t(d);
+        }
+    }
+    tileSync<Waves>();
+#pragma unroll 1
+    for (uint32_t k = 0; k < chunks; k++) {
+        const uint32_t r = sh.chunk[k] + tid;
+        const bool mine = r < sh.chunk[k + 1];
+        bool emits = false;
+        if (mine) {
+            const uint32_t m = sh.meta[r], first = metaFirst(m);
+            const uint32_t n = uint32_t(__builtin_popcount(metaInner(m)));
+            emits = metaEmits(m) != 0u;
+            uint32_t d = (sh.aux[r] & 0xffffu) + 1u, a[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                a[j] = j < n ? sh.aux[first + j] : 0u;
+#pragma unroll
+            for (uint32_t j = 4; j-- > 0;)
+                if (j < n) {
+                    sh.aux[first + j] = (a[j] & 0xffff0000u) | d;
+                    d += a[j] & 0xffffu;
+                }
+        }
+        // the emitting records' list, in any order, in the low bits of the metas of
+        // records that lie before this chunk's end (whose `first` has been read)
+        const uint64_t be = ballot(emits);
+        uint32_t at = 0;
+        if (lane == 0 && be != 0ull)
+            at = atomicAdd(&sh.emitters, uint32_t(__builtin_popcountll(be)));
+        at = readLane(at, 0) + lanesBelow(be);
+        tileSync<Waves>();
+        if (emits)
+            sh.meta[at] = (sh.meta[at] & 0xfff00000u) | r;
+    }
+    tileSync<Waves>();
+    const uint32_t nEmit = uniform(sh.emitters);
+    if (nEmit > ElemCap)
+        return give(TileResult::TooBig);
+    constexpr uint32_t K = (ElemCap + T - 1) / T; // elements per thread
+    bad = false;
+    if (rank) {
+        uint32_t at[K], rec[K];
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++) {
+            at[k] = rec[k] = 0;
+            if (k * T + tid < nEmit) {
+                rec[k] = metaFirst(sh.meta[k * T + tid]);
+                for (uint32_t i = 0; i < nEmit; i++)
+                    at[k] += visitedBefore(sh, metaFirst(sh.meta[i]), rec[k], families, n0, bs) ? 1u : 0u;
+            }
+        }
+        tileSync<Waves>();
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++)
+            if (k * T + tid < nEmit)
+                sh.elem[at[k]].w = rec[k];
+    } else {
+        // the elements take the place of the keys and aux words: through registers
+        uint4 e[K];
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++) {
+            const uint32_t i = k * T + tid;
+            if (i < nEmit) {
+                const uint32_t r = metaFirst(sh.meta[i]), a = sh.aux[r], rp = a >> 16;
+                e[k].x = orderedKey(bitsf(sh.key[r]));
+                if (rp == kNoRecord) {
+                    e[k].y = kOldest;
+                    e[k].z = 0xffff0000u | (a & 0xffffu);
+                    e[k].w = 0xffff0000u | r;
+                } else {
+                    const uint32_t p = sh.aux[rp];
+                    e[k].y = ~orderedKey(bitsf(sh.key[rp]));
+                    e[k].z = (~p << 16) | (a & 0xffffu);
+                    e[k].w = (p & 0xffff0000u) | r;
+                }
+            }
+        }
+        tileSync<Waves>();
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++)
+            if (k * T + tid < nEmit)
+                sh.elem[k * T + tid] = e[k];
+        sortElements<Cfg>(sh, nEmit, tid);
+#pragma unroll 1
+        for (uint32_t i = tid + 1u; i < nEmit; i += T) {
+            const uint4 a = sh.elem[i - 1u], b = sh.elem[i];
+            bad |= a.x == b.x && a.y == b.y && (a.z ^ b.z) > 0xffffu && (a.w ^ b.w) > 0xffffu;
+        }
+        if (families) {
+            tileSync<Waves>();
+#pragma unroll 1
+            for (uint32_t i = tid; i < nEmit; i += T) {
+                uint4 e = sh.elem[i];
+                const uint32_t q = familyOf(sh, n0, e.z & 0xffffu), key = orderedKey(bs[q].tMin);
+                if (e.x > key) {
+                    const uint32_t wp = ~e.y;
+                    e.y = ~(wp > key ? wp : key);
+                } else {
+                    e.x = key;
+                    e.y = kUncovered | (63u - q);
+                }
+                e.z = (i << 8) | q;
+                sh.elem[i] = e;
+            }
+            sortElements<Cfg>(sh, nEmit, tid);
+#pragma unroll 1
+            for (uint32_t i = tid + 1u; i < nEmit; i += T) {
+                const uint4 a = sh.elem[i - 1u], b = sh.elem[i];
+                bad |= a.x == b.x && a.y == b.y && a.y < kUncovered && ((a.z ^ b.z) & 0xffu) != 0u;
+            }
+        }
+    }
+    if (ballot(bad) != 0ull && lane == 0)
+        sh.bad = 1u;
+    tileSync<Waves>(); // the elements have been compared
+
+    // ---- phase C: emit ----
+    // each record's list length, then its place, into its element
+    auto leafRanges = [&](uint32_t i, uint32_t& leaf, uint32_t d[5]) {
+        const uint32_t r = sh.elem[i].w & 0xffffu;
+        leaf = metaEmits(sh.meta[r]);
+        const uint32_t* data = nodes[sh.node[r]].data;
+#pragma unroll
+        for (int k = 0; k < 5; k++)
+            d[k] = data[k];
+    };
+    uint32_t sum = 0;
+#pragma unroll 1
+    for (uint32_t i = tid; i < nEmit; i += T) {
+        uint32_t leaf, d[5], len = 0;
+        leafRanges(i, leaf, d);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if ((leaf & (1u << k)) && d[k + 1] > d[k])
+                len += d[k + 1] - d[k];
+        sh.elem[i].x = len;
+        sum += len;
+    }
+    sum = waveSum(sum);
+    uint64_t start = 0;
+    bool fits = true;
+    if constexpr (Waves > 1) {
+        if (lane == 0)
+            sh.waveTotals[wave] = sum;
+        __syncthreads();
+        if (uniform(sh.bad) != 0u)
+            return give(TileResult::Undecided);
+        if (wave == 0) {
+            const uint32_t total = waveSum(lane < Waves ? sh.waveTotals[lane] : 0u);
+            start = claimList(g, tile, total, nrec, n0, lane, fits);
+            if (lane == 0) {
+                sh.listStart[0] = uint32_t(start);
+                sh.listStart[1] = uint32_t(start >> 32);
+                sh.listFits = fits ? 1u : 0u;
+                g.tileLevel[tile] = levelFor(nrec);
+            }
+        }
+        __syncthreads();
+        start = uniform(sh.listStart[0]);
+        fits = uniform(sh.listFits) != 0u;
+    } else {
+        waveLdsSync();
+        if (uniform(sh.bad) != 0u)
+            return give(TileResult::Undecided);
+        start = claimList(g, tile, sum, nrec, n0, lane, fits);
+    }
+    if (!fits)
+        return TileResult::Done;
+    uint32_t run = uint32_t(start);
+#pragma unroll 1
+    for (uint32_t base = 0; base < nEmit; base += 64) {
+        // (every wave sums every block's lengths and writes its own blocks)
+        const uint32_t i = base + lane;
+        const uint32_t len = i < nEmit ? sh.elem[i].x : 0u;
+        const uint32_t incl = waveInclusiveScan(len);
+        uint32_t at = run + incl - len;
+        run += readLane(incl, 63);
+        if ((Waves == 1 || (base / 64) % Waves == wave) && len != 0u) {
+            uint32_t leaf, d[5];
+            leafRanges(i, leaf, d);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (leaf & (1u << k))
+#pragma unroll 1
+                    for (uint32_t t = d[k]; t < d[k + 1]; t++)
+                        g.triOut[at++] = t;
+        }
+    }
+    return TileResult::Done;
+}
+
+// a tile of a configuration's launch; one it cannot hold is queued for the next
+// configuration, an irregular one for the colossal configuration's serial walk
+template <class Cfg>
+__device__ inline void tileListOne(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t tile, uint32_t tid) {
+    TileResult r = TileResult::Undecided;
+    for (uint32_t attempt = 0; attempt < 2u && r == TileResult::Undecided; attempt++) {
+        tileSync<Cfg::Waves>(); // the previous tile's (or attempt's) LDS reads are done
+        r = tileListBody<Cfg>(g, sh, tile, tid, attempt != 0u);
+    }
+    if (r != TileResult::Done && tid == 0) {
+        const uint32_t skip = r == TileResult::Irregular ? uint32_t(TileListColossal::Level) - 1u - Cfg::Level : 0u;
+        const unsigned long long slot = atomicAdd(&g.counters[g.nextCounter + skip], 1ull);
+        g.nextQueue[size_t(skip) * g.tileCount + slot] = tile;
+    }
+}
+
+// A tile whose last list on this scene needed a still bigger configuration than `level`
+// goes straight to that one's queue (queue h - 1, its length in counters[4 + h]). The
+// standard configuration takes every tile first and keeps no hints. Hints are 0 (none) or
+// 1..5; anything else is ignored.
+__device__ inline bool followHint(const TileListArgs& g, uint32_t level, uint32_t tile, uint32_t tid) {
+    const uint32_t hint = g.useHints ? uniform(g.tileLevel[tile]) : 0u;
+    if (hint <= level || hint > 5u)
+        return false;
+    if (tid == 0) {
+        const unsigned long long slot = atomicAdd(&g.counters[4 + hint], 1ull);
+        g.nextQueue[size_t(hint - 1u - level) * g.tileCount + slot] = tile;
+    }
+    return true;
+}
+
+// every tile, standard configuration
+__global__ __launch_bounds__(64) void tileListKernel(TileListArgs g) {
+    __shared__ TileListLds<TileListSmall> sh;
+    tileListOne(g, sh, blockIdx.x, threadIdx.x);
+}
+
+__global__ __launch_bounds__(64) void tileListBatchKernel(const TileListArgs* __restrict__ all,
+                                                          const uint32_t* __restrict__ start, uint32_t n,
+                                                          uint32_t swizzle) {
+    __shared__ TileListLds<TileListSmall> sh;
+    const uint32_t unit = xcdUnit(blockIdx.x, gridDim.x, swizzle);
+    const uint32_t v = batchView(start, n, unit);
+    tileListOne(batchArgs(all, v), sh, unit - start[v], threadIdx.x);
+}
+
+// The tiles a smaller configuration queued, persistent workgroups: this workgroup takes
+// the entries `first`, `first` + stride, ... of the queue.
+template <class Cfg>
+__device__ inline void tileListQueueRun(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t first, uint32_t stride,
+                                        uint32_t queued, uint32_t tid) {
+    for (uint32_t i = first; i < queued; i += stride) {
+        const uint32_t tile = uniform(g.queue[i]);
+        if (followHint(g, Cfg::Level, tile, tid))
+            continue;
+        tileListOne(g, sh, tile, tid);
+    }
+}
+
+template <class Cfg>
+__global__ __launch_bounds__(64 * Cfg::Waves) __attribute__((amdgpu_waves_per_eu(Cfg::Occupancy)))
+void tileListQueueKernel(TileListArgs g) {
+    __shared__ TileListLds<Cfg> sh;
+    const uint32_t queued = uniform(uint32_t(g.counters[g.queueCounter]));
+    tileListQueueRun<Cfg>(g, sh, blockIdx.x, gridDim.x, queued, threadIdx.x);
+}
+
+// every view's queue in turn, the entries of all of them dealt to the workgroups as one
+// sequence
+template <class Cfg>
+__global__ __launch_bounds__(64 * Cfg::Waves) __attribute__((amdgpu_waves_per_eu(Cfg::Occupancy)))
+void tileListQueueBatchKernel(const TileListArgs* __restrict__ all,
+                                                                            uint32_t n) {
+    __shared__ TileListLds<Cfg> sh;
+    uint32_t base = 0;
+    for (uint32_t v = 0; v < n; v++) {
+        const TileListArgs& g = all[v];
+        const uint32_t queued = uniform(uint32_t(g.counters[g.queueCounter]));
+        const uint32_t first = (blockIdx.x + gridDim.x - base % gridDim.x) % gridDim.x;
+        tileListQueueRun<Cfg>(g, sh, first, gridDim.x, queued, threadIdx.x);
+        base += queued;
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// Colossal configuration: the walk replayed over the records by one wave, for the tiles
+// whose records outgrow the sort's configurations and the irregular ones.
+// The tests run as in phase A. Then the reference's distance-sorted stack walk is replayed
+// over the records with the stack in registers (reg_stack.h): pops, the single-child
+// shortcut, the sorted insertion (one ballot per register finds the position, two DPP
+// shifts per register move the entries above it), and the sequence of records whose leaves
+// are emitted. Records none of whose subtree emits are left out: the reference pops them
+// and does nothing else. Its stack stays sorted by key, ties newest on top (the block stack
+// arrives sorted and every insert lands at its sorted position), so a pop always takes the
+// least (key, newest) entry; an entry that changes nothing when popped can be dropped
+// without moving any other pop. A NaN key breaks that order (it inserts on top of anything),
+// so a tile with a NaN or infinite key, or with an unsorted block stack, goes to the
+// LDS-stack walk, as does a tile whose records or stack exceed the capacity.
+// ---------------------------------------------------------------------------------
+struct TileSerialLds {
+    uint32_t recKey[TileListColossal::RecCap];  // float bits of the record's distance key; in the
+                                                // emission, the list length of emitted record i
+    uint32_t recMeta[TileListColossal::RecCap]; // packMeta
+};
 
 // Builds one tile's list; false when the tile does not fit this configuration (its count
 // and offset are then zero).
-template <class Cfg>
-__device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t tile, uint32_t lane) {
-    using Stack = typename Cfg::Stack;
+__device__ bool tileSerialBody(const TileListArgs& g, TileSerialLds& sh, uint32_t tile, uint32_t lane) {
+    using Cfg = TileListColossal;
+    using Stack = Cfg::Stack;
     const BVHNode* __restrict__ nodes = g.nodes;
     const uint32_t block = tile / TILES_PER_BLOCK;
     const FrustumPre* __restrict__ f = g.tilePre + tile;
@@ -392,45 +1104,10 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
         }
         return true;
     }
-    if constexpr (Cfg::Level > 0) {
-        // A tile whose last list on this scene needed a still bigger configuration goes
-        // straight to that one's queue (queue h - 1, its length in counters[4 + h]). The
-        // standard configuration takes every tile first and keeps no hints: its code stays
-        // as short as it is. Hints are 0 (none) or 1..5; anything else is ignored.
-        const uint32_t hint = g.useHints ? g.tileLevel[tile] : 0u;
-        if (hint > uint32_t(Cfg::Level) && hint <= 5u) {
-            if (lane == 0) {
-                const unsigned long long slot = atomicAdd(&g.counters[4 + hint], 1ull);
-                g.nextQueue[size_t(hint - 1u - Cfg::Level) * g.tileCount + slot] = tile;
-            }
-            return true;
-        }
-    }
-    uint32_t* gNode = nullptr; // the record node indices and emission order outside LDS
-    uint16_t* gOrder = nullptr;
-    if constexpr (!Cfg::LdsRecords) {
-        gNode = g.recScratch + size_t(blockIdx.x) * recScratchWords<Cfg>();
-        gOrder = reinterpret_cast<uint16_t*>(gNode + Cfg::RecCap);
-    }
-    auto recNode = [&](uint32_t i) -> uint32_t& {
-        if constexpr (Cfg::LdsRecords)
-            return sh.recNode[i];
-        else
-            return gNode[i];
-    };
-    // the emission order: entry i is the i-th record whose leaves are emitted
-    auto order = [&](uint32_t i) -> uint32_t {
-        if constexpr (Cfg::LdsRecords)
-            return (sh.recMeta[i] >> 10) & 0x3ffu;
-        else
-            return gOrder[i];
-    };
-    auto setOrder = [&](uint32_t i, uint32_t rec) {
-        if constexpr (Cfg::LdsRecords)
-            sh.recMeta[i] = (sh.recMeta[i] & ~(0x3ffu << 10)) | (rec << 10);
-        else
-            gOrder[i] = uint16_t(rec);
-    };
+    // the record node indices and the emission order outside LDS (entry i: the i-th record
+    // whose leaves are emitted)
+    uint32_t* recNode = g.recScratch + size_t(blockIdx.x) * recScratchWords();
+    uint16_t* order = reinterpret_cast<uint16_t*>(recNode + Cfg::RecCap);
     const uint32_t limit = g.stackLimit < uint32_t(Cfg::StackCap) ? g.stackLimit : uint32_t(Cfg::StackCap);
     bool overflow = n0 > limit;
     uint32_t deepest = n0; // deepest stack size seen
@@ -443,7 +1120,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
         bool nanKey = false;
         if (lane < n0) {
             StackEntry e = bs[lane];
-            recNode(lane) = e.nodeMask & STACK_NODE_MASK;
+            recNode[lane] = e.nodeMask & STACK_NODE_MASK;
             sh.recKey[lane] = fbits(e.tMin);
             sh.recMeta[lane] = packMeta(0u, 0u, 0u, e.nodeMask >> 28);
             nanKey = !(fabsf(e.tMin) <= FLT_MAX); // NaN or infinite
@@ -467,7 +1144,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
                 nodeR[k] = 0;
                 entryR[k] = 0;
                 if (valid[k]) {
-                    nodeR[k] = recNode(recI[k]);
+                    nodeR[k] = recNode[recI[k]];
                     entryR[k] = metaEntry(sh.recMeta[recI[k]]);
                 }
             }
@@ -475,58 +1152,8 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
 #pragma unroll
             for (uint32_t k = 0; k < S; k++)
                 X[k] = loadChildBox(nodes, nodeR[k], c, axis);
-            // (`&` rather than `&&` throughout: no branch per lane condition)
-            bool pass[S], refine[S];
-            uint64_t need[S];
-            uint32_t nNeed = 0;
-#pragma unroll
-            for (uint32_t k = 0; k < S; k++) {
-                pass[k] = valid[k] & childCoarsePass(f, X[k].b0, X[k].b1, X[k].b2, X[k].b3, X[k].b4, X[k].b5);
-                const uint32_t m = uint32_t(ballot(pass[k]) >> (4 * s)) & 0xfu;
-                // refine only nodes with a passing leaf child (traverse_avx.h:447-452)
-                refine[k] = pass[k] & ((m & X[k].leafMask) != 0u);
-                need[k] = ballot(refine[k]);
-                nNeed += uint32_t(__builtin_popcountll(need[k]));
-            }
-            if (nNeed != 0u) {
-                if (nNeed < 64u) {
-                    // Few boxes need the 12-axis test (typically a sixth of the lanes): move
-                    // them to lanes 0 .. nNeed - 1 with forward permutes (every other lane
-                    // sends to lane 63, which then holds no needed box), test them in one
-                    // pass, and read each verdict back from the ballot.
-                    uint32_t d[S];
-                    float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f, g3 = 0.0f, g4 = 0.0f, g5 = 0.0f;
-                    uint32_t base = 0;
-#pragma unroll
-                    for (uint32_t k = 0; k < S; k++) {
-                        const uint32_t nk = uint32_t(__builtin_popcountll(need[k]));
-                        d[k] = refine[k] ? base + lanesBelow(need[k]) : 63u;
-                        const bool mine = lane >= base && lane < base + nk; // slot k's boxes land here
-                        auto take = [&](float& gq, float v) {
-                            const uint32_t x = uint32_t(__builtin_amdgcn_ds_permute(int(d[k] << 2), int(fbits(v))));
-                            gq = mine ? bitsf(x) : gq;
-                        };
-                        take(g0, X[k].b0);
-                        take(g1, X[k].b1);
-                        take(g2, X[k].b2);
-                        take(g3, X[k].b3);
-                        take(g4, X[k].b4);
-                        take(g5, X[k].b5);
-                        base += nk;
-                    }
-                    const bool cull = childRefineCull(f, g0, g1, g2, g3, g4, g5);
-                    const uint64_t culled = ballot(cull & (lane < nNeed));
-#pragma unroll
-                    for (uint32_t k = 0; k < S; k++)
-                        pass[k] &= !(refine[k] & (((culled >> d[k]) & 1ull) != 0ull));
-                } else {
-#pragma unroll
-                    for (uint32_t k = 0; k < S; k++) {
-                        const bool cullK = childRefineCull(f, X[k].b0, X[k].b1, X[k].b2, X[k].b3, X[k].b4, X[k].b5);
-                        pass[k] &= !(refine[k] & cullK);
-                    }
-                }
-            }
+            bool pass[S];
+            testChildBoxes<S>(stepFrustum(f), X, valid, lane, pass);
             // internal children are pushed only from entries without a leaf mask
             // (traverse_avx.h:476-483); slot k's children follow those of slots below it
             uint32_t before = 0;
@@ -538,7 +1165,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
                 const uint64_t bi = ballot(inner);
                 const uint32_t slot = nrec + before + lanesBelow(bi);
                 if (inner && slot < Cfg::RecCap) {
-                    recNode(slot) = nodeR[k] + X[k].childOffset;
+                    recNode[slot] = nodeR[k] + X[k].childOffset;
                     sh.recKey[slot] = fbits(X[k].key);
                     sh.recMeta[slot] = 0u;
                 }
@@ -575,7 +1202,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
             const uint32_t meta = valid ? sh.recMeta[r] : 0u;
             const uint32_t mask = metaMask(meta), leaf = metaLeaf(meta);
             const uint32_t inner = metaEntry(meta) == 0u ? mask & ~leaf : 0u;
-            const uint32_t first = metaFirst<Cfg>(meta);
+            const uint32_t first = metaFirst(meta);
             const uint32_t nInner = uint32_t(__builtin_popcount(inner));
             // emitting records keep their mask; the others keep it while a child is live
             bool open = valid && mask != 0u && (mask & leaf) == 0u;
@@ -614,7 +1241,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
             const uint32_t dest = ((live >> lane) & 1u) ? lanesBelow(live) : size + lanesBelow(~live);
             const float t = bitsf(uint32_t(__builtin_amdgcn_ds_permute(int(dest << 2), int(key))));
             const uint32_t m =
-                uint32_t(__builtin_amdgcn_ds_permute(int(dest << 2), int(stackEntry<Cfg>(lane, meta))));
+                uint32_t(__builtin_amdgcn_ds_permute(int(dest << 2), int(lane)));
             stackInit(st, t, m, size, lane);
             const float above = __shfl_down(t, 1);
             if (ballot(lane + 1u < size && t < above) != 0ull)
@@ -624,9 +1251,13 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
         uint32_t emitBuf = 0; // emission order, 64 records at a time
         uint32_t steps = 0;
         uint32_t curRec = 0, curMeta = 0;
+        auto popRecord = [&] {
+            curRec = stackPop(st, lane);
+            curMeta = uniform(sh.recMeta[curRec]);
+        };
         bool walking = !overflow && st.size != 0u;
         if (walking)
-            fromStackEntry<Cfg>(stackPop(st, lane), sh, curRec, curMeta);
+            popRecord();
         while (walking) {
             // every record is reached at most once; the bound keeps the loop finite whatever
             // the records hold
@@ -639,7 +1270,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
                 emitBuf = writeLane(emitBuf, curRec, nEmit & 63u, lane);
                 nEmit++;
                 if ((nEmit & 63u) == 0u)
-                    setOrder(nEmit - 64u + lane, emitBuf);
+                    order[nEmit - 64u + lane] = uint16_t(emitBuf);
             }
             // internal children are followed only from entries without a leaf mask
             const uint32_t inner = metaEntry(curMeta) == 0u ? mask & ~leafMask : 0u;
@@ -649,7 +1280,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
             if (inner != 0u) {
                 // the hit children's records, contiguous from `first` in child order; lanes
                 // past them read an in-range record and are masked off
-                const uint32_t first = metaFirst<Cfg>(curMeta);
+                const uint32_t first = metaFirst(curMeta);
                 const uint32_t nChildren = uint32_t(__builtin_popcount(inner));
                 const uint32_t r = first + lane < uint32_t(Cfg::RecCap) ? first + lane : uint32_t(Cfg::RecCap) - 1u;
                 const uint32_t childKey = sh.recKey[r];
@@ -687,7 +1318,7 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
                     const uint32_t best = 31u - uint32_t(__builtin_clz(atLeast));
                     const float bestKey = bitsf(readLane(fbits(least), 0));
                     const bool take = st.size == 0u || bestKey <= stackTopKey(st);
-                    const uint32_t entry = stackEntry<Cfg>(first + lane, childMeta);
+                    const uint32_t entry = first + lane;
                     // at most four siblings: straight-line code (a loop here keeps the
                     // compiler from holding the stack in the same registers on every path)
                     uint32_t sib = liveBits & ~(take ? 1u << best : 0u);
@@ -711,11 +1342,11 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
             if (pop) {
                 if (st.size == 0u)
                     break;
-                fromStackEntry<Cfg>(stackPop(st, lane), sh, curRec, curMeta);
+                popRecord();
             }
         }
         if (!overflow && (nEmit & 63u) != 0u && lane < (nEmit & 63u))
-            setOrder((nEmit & ~63u) + lane, emitBuf);
+            order[(nEmit & ~63u) + lane] = uint16_t(emitBuf);
         waveLdsSync();
     }
     if (overflow) {
@@ -736,10 +1367,10 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
         const uint32_t i = base + lane;
         uint32_t len = 0;
         if (i < nEmit) {
-            const uint32_t rec = order(i);
+            const uint32_t rec = order[i];
             const uint32_t meta = sh.recMeta[rec];
             const uint32_t leaf = metaMask(meta) & metaLeaf(meta);
-            const uint32_t* d = nodes[recNode(rec)].data;
+            const uint32_t* d = nodes[recNode[rec]].data;
             uint32_t dk[5];
 #pragma unroll
             for (int k = 0; k < 5; k++)
@@ -765,28 +1396,10 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
             total += waveSum(len);
         }
     }
-    unsigned long long start = 0;
+    bool fits = true;
+    const uint64_t start = claimList(g, tile, total, nrec, deepest, lane, fits);
     if (lane == 0)
-        start = atomicAdd(&g.counters[3], (unsigned long long)total);
-    start = (uint64_t(readLane(uint32_t(start >> 32), 0)) << 32) | readLane(uint32_t(start), 0);
-    const bool fits = start + total <= g.capacity;
-    if (lane == 0) {
-        g.counts[tile] = total;
-        g.offsets[tile] = uint32_t(start);
-        if (!fits)
-            atomicOr(&g.counters[1], 1ull);
-        g.tileWork[tile] = nrec; // node visits
-        g.tileWork[g.tileCount + tile] = deepest;
-        if constexpr (Cfg::Level > 0) {
-            // the smallest queued configuration this tile's records and stack fit, for its
-            // next frame
-            const uint32_t level = nrec <= TileListLarge::RecCap && deepest <= REG_STACK4_CAP    ? 1u
-                                   : nrec <= TileListHuge::RecCap && deepest <= REG_STACK8_CAP   ? 2u
-                                   : nrec <= TileListGiant::RecCap ? 3u
-                                                                   : 4u;
-            g.tileLevel[tile] = level;
-        }
-    }
+        g.tileLevel[tile] = levelFor(nrec);
     if (!fits)
         return true;
     {
@@ -807,10 +1420,10 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
         uint32_t at = run + incl - len;
         run += readLane(incl, 63);
         if (len) {
-            const uint32_t rec = order(i);
+            const uint32_t rec = order[i];
             const uint32_t meta = sh.recMeta[rec];
             const uint32_t leaf = metaMask(meta) & metaLeaf(meta);
-            const uint32_t* d = nodes[recNode(rec)].data;
+            const uint32_t* d = nodes[recNode[rec]].data;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const uint32_t t0 = d[k], t1 = d[k + 1];
@@ -823,68 +1436,34 @@ __device__ bool tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32
     return true;
 }
 
-// every tile, standard configuration; a tile it cannot hold is queued for the large one
-__device__ inline void tileListSmallOne(const TileListArgs& g, TileListLds<TileListSmall>& sh, uint32_t tile,
-                                        uint32_t lane) {
-    if (!tileListBody<TileListSmall>(g, sh, tile, lane) && lane == 0) {
-        const unsigned long long slot = atomicAdd(&g.counters[g.nextCounter], 1ull);
-        g.nextQueue[slot] = tile;
-    }
-}
-
-// The LDS records (680 x 12 bytes, 8160 bytes: the emission order shares the metas' words)
-// let a CU hold 20 of these waves. A record capacity below what a scene's densest tiles
-// need costs more than the waves it adds: the tiles it sends to the large configuration
-// run after this kernel, each a serial walk of one wave (the densest tile of the stereo
-// room eye holds 652 records).
-__global__ __launch_bounds__(64) void tileListKernel(TileListArgs g) {
-    __shared__ TileListLds<TileListSmall> sh;
-    tileListSmallOne(g, sh, blockIdx.x, threadIdx.x);
-}
-
-__global__ __launch_bounds__(64) void tileListBatchKernel(const TileListArgs* __restrict__ all,
-                                                          const uint32_t* __restrict__ start, uint32_t n,
-                                                          uint32_t swizzle) {
-    __shared__ TileListLds<TileListSmall> sh;
-    const uint32_t unit = xcdUnit(blockIdx.x, gridDim.x, swizzle);
-    const uint32_t v = batchView(start, n, unit);
-    tileListSmallOne(batchArgs(all, v), sh, unit - start[v], threadIdx.x);
-}
-
-// The tiles a smaller configuration queued, persistent workgroups: this workgroup takes
-// the entries `first`, `first` + stride, ... of the queue; a tile this configuration
-// cannot hold either is queued for the next.
-template <class Cfg>
-__device__ inline void tileListQueueRun(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t first, uint32_t stride,
-                                        uint32_t queued, uint32_t lane) {
+__device__ inline void tileSerialRun(const TileListArgs& g, TileSerialLds& sh, uint32_t first, uint32_t stride,
+                                     uint32_t queued, uint32_t lane) {
     for (uint32_t i = first; i < queued; i += stride) {
         const uint32_t tile = uniform(g.queue[i]);
+        if (followHint(g, TileListColossal::Level, tile, lane))
+            continue;
         waveLdsSync(); // the previous tile's LDS reads are done
-        if (!tileListBody<Cfg>(g, sh, tile, lane) && lane == 0) {
+        if (!tileSerialBody(g, sh, tile, lane) && lane == 0) {
             const unsigned long long slot = atomicAdd(&g.counters[g.nextCounter], 1ull);
             g.nextQueue[slot] = tile;
         }
     }
 }
 
-template <class Cfg>
-__global__ __launch_bounds__(64) void tileListQueueKernel(TileListArgs g) {
-    __shared__ TileListLds<Cfg> sh;
+__global__ __launch_bounds__(64) void tileSerialKernel(TileListArgs g) {
+    __shared__ TileSerialLds sh;
     const uint32_t queued = uniform(uint32_t(g.counters[g.queueCounter]));
-    tileListQueueRun<Cfg>(g, sh, blockIdx.x, gridDim.x, queued, threadIdx.x);
+    tileSerialRun(g, sh, blockIdx.x, gridDim.x, queued, threadIdx.x);
 }
 
-// every view's queue in turn, the entries of all of them dealt to the workgroups as one
-// sequence
-template <class Cfg>
-__global__ __launch_bounds__(64) void tileListQueueBatchKernel(const TileListArgs* __restrict__ all, uint32_t n) {
-    __shared__ TileListLds<Cfg> sh;
+__global__ __launch_bounds__(64) void tileSerialBatchKernel(const TileListArgs* __restrict__ all, uint32_t n) {
+    __shared__ TileSerialLds sh;
     uint32_t base = 0;
     for (uint32_t v = 0; v < n; v++) {
         const TileListArgs& g = all[v];
         const uint32_t queued = uniform(uint32_t(g.counters[g.queueCounter]));
         const uint32_t first = (blockIdx.x + gridDim.x - base % gridDim.x) % gridDim.x;
-        tileListQueueRun<Cfg>(g, sh, first, gridDim.x, queued, threadIdx.x);
+        tileSerialRun(g, sh, first, gridDim.x, queued, threadIdx.x);
         base += queued;
     }
 }
@@ -1022,21 +1601,17 @@ __device__ inline void tileWalkOne(const TileWalkArgs& a, TileWalkLds& sh, uint3
                 a.offsets[tile] = uint32_t(start);
                 if (start + count > capacity)
                     atomicOr(&counters[1], 1ull);
-                // the smallest queued configuration whose records and stack would hold this
-                // walk (the walk's stack is the unpruned one, never shallower), unless the
-                // tile can only be walked
-                // (with a view stack limit below 64 every configuration has that limit)
+                // the smallest queued configuration whose records would hold this walk, unless
+                // the tile can only be walked (an irregular one, one over the view's stack
+                // limit, one whose walk outgrows the colossal configuration; the walk's
+                // stack is the unpruned one, never shallower)
                 const bool full = a.stackLimit >= REG_STACK_CAP;
-                const uint32_t capL = full ? REG_STACK4_CAP : a.stackLimit;
-                const uint32_t capH = full ? REG_STACK8_CAP : a.stackLimit;
-                const uint32_t capG = full ? REG_STACK16_CAP : a.stackLimit;
-                const uint32_t capC = full ? REG_STACK16_CAP : a.stackLimit;
-                a.tileLevel[tile] = irregular                                               ? 5u
-                                    : visits <= TileListLarge::RecCap && maxSize <= capL    ? 1u
-                                    : visits <= TileListHuge::RecCap && maxSize <= capH     ? 2u
-                                    : visits <= TileListGiant::RecCap && maxSize <= capG    ? 3u
-                                    : visits <= TileListColossal::RecCap && maxSize <= capC ? 4u
-                                                                                            : 5u;
+                const uint32_t level = levelFor(visits);
+                const bool walkOnly = irregular || n0 > a.stackLimit ||
+                                      (level == TileListColossal::Level &&
+                                       (visits > TileListColossal::RecCap ||
+                                        maxSize > (full ? uint32_t(REG_STACK16_CAP) : a.stackLimit)));
+                a.tileLevel[tile] = walkOnly ? 5u : level;
                 a.tileWork[tile] = visits; // node visits
                 a.tileWork[a.tileCount + tile] = maxSize;
             }
@@ -1217,6 +1792,7 @@ TileListArgs tileListArgs(const hvvr_gpu_view* v, const hvvr_gpu_scene* s, int l
     TileListArgs g;
     g.nodes = s->nodes.ptr;
     g.tilePre = v->tilePre.ptr;
+    g.blockPre = v->blockPre.ptr;
     g.blockStacks = v->blockStacks.ptr;
     g.blockStackSize = v->blockStackSize.ptr;
     g.counts = v->tileCounts.ptr;
@@ -1225,15 +1801,14 @@ TileListArgs tileListArgs(const hvvr_gpu_view* v, const hvvr_gpu_scene* s, int l
     g.capacity = v->listCapacity;
     g.counters = reinterpret_cast<unsigned long long*>(v->counters.ptr);
     // level L takes queue L - 1 (counters[4 + L]) and fills queue L (counters[5 + L]); the
-    // larger configurations' stack limit is the view's limit scaled past the standard one
-    // (a test limit below 64 keeps every configuration short)
+    // stack limit bounds the block stack (at most 64 entries) and the serial walk's stack
+    // (a limit below 64 sends deeper tiles to the LDS-stack walk)
     g.queue = level > 0 ? queues + (level - 1) * T : nullptr;
     g.queueCounter = level > 0 ? uint32_t(4 + level) : 0u;
     g.nextQueue = queues + level * T;
     g.nextCounter = uint32_t(5 + level);
     const bool full = v->waveStackLimit >= REG_STACK_CAP;
-    const uint32_t caps[5] = {v->waveStackLimit, REG_STACK4_CAP, REG_STACK8_CAP, REG_STACK16_CAP, REG_STACK16_CAP};
-    g.stackLimit = level == 0 || !full ? v->waveStackLimit : caps[level];
+    g.stackLimit = full && level == int(TileListColossal::Level) ? uint32_t(REG_STACK16_CAP) : v->waveStackLimit;
     g.recScratch = v->recScratch.ptr;
     g.tileLevel = v->tileLevel.ptr;
     g.useHints = v->hintScene == s ? 1u : 0u;
@@ -1246,20 +1821,13 @@ static uint32_t clampGroups(uint32_t want, uint32_t tiles) {
     return want < tiles ? want : (tiles ? tiles : 1u);
 }
 
-size_t tileListScratchWords() {
-    const size_t large = size_t(kMaxLargeGroups) * recScratchWords<TileListLarge>();
-    const size_t huge = size_t(kMaxHugeGroups) * recScratchWords<TileListHuge>();
-    const size_t giant = size_t(kMaxGiantGroups) * recScratchWords<TileListGiant>();
-    const size_t colossal = size_t(kMaxColossalGroups) * recScratchWords<TileListColossal>();
-    return std::max(std::max(large, huge), std::max(giant, colossal));
-}
+size_t tileListScratchWords() { return size_t(kMaxColossalGroups) * recScratchWords(); }
 
 void tileListGroupsFor(size_t words, uint32_t groups[4]) {
-    const size_t per[4] = {recScratchWords<TileListLarge>(), recScratchWords<TileListHuge>(),
-                           recScratchWords<TileListGiant>(), recScratchWords<TileListColossal>()};
-    const uint32_t most[4] = {kMaxLargeGroups, kMaxHugeGroups, kMaxGiantGroups, kMaxColossalGroups};
-    for (int k = 0; k < 4; k++)
-        groups[k] = uint32_t(std::min<size_t>(most[k], words / per[k]));
+    groups[0] = kMaxLargeGroups;
+    groups[1] = kMaxHugeGroups;
+    groups[2] = kMaxGiantGroups;
+    groups[3] = uint32_t(std::min<size_t>(kMaxColossalGroups, words / recScratchWords()));
 }
 
 // the arguments of configuration `level` with the record scratch and queues of `scratch`
@@ -1288,12 +1856,13 @@ void launchTileLists(hvvr_gpu_view* v, const hvvr_gpu_scene* s, hipStream_t stre
                               tileListArgsWith(v, s, 0, scratch));
     else
         tileListKernel<<<T, 64, 0, stream>>>(tileListArgsWith(v, s, 0, scratch));
-    // 16 KB of LDS: ten workgroups per CU; 36 KB: four; 80 KB: two; 160 KB: one
-    tileListQueueKernel<TileListLarge><<<clampGroups(large, T), 64, 0, stream>>>(tileListArgsWith(v, s, 1, scratch));
-    tileListQueueKernel<TileListHuge><<<clampGroups(huge, T), 64, 0, stream>>>(tileListArgsWith(v, s, 2, scratch));
-    tileListQueueKernel<TileListGiant><<<clampGroups(giant, T), 64, 0, stream>>>(tileListArgsWith(v, s, 3, scratch));
-    tileListQueueKernel<TileListColossal>
-        <<<clampGroups(colossal, T), 64, 0, stream>>>(tileListArgsWith(v, s, 4, scratch));
+    tileListQueueKernel<TileListLarge>
+        <<<clampGroups(large, T), 64 * TileListLarge::Waves, 0, stream>>>(tileListArgsWith(v, s, 1, scratch));
+    tileListQueueKernel<TileListHuge>
+        <<<clampGroups(huge, T), 64 * TileListHuge::Waves, 0, stream>>>(tileListArgsWith(v, s, 2, scratch));
+    tileListQueueKernel<TileListGiant>
+        <<<clampGroups(giant, T), 64 * TileListGiant::Waves, 0, stream>>>(tileListArgsWith(v, s, 3, scratch));
+    tileSerialKernel<<<clampGroups(colossal, T), 64, 0, stream>>>(tileListArgsWith(v, s, 4, scratch));
 }
 
 void launchTileListFallback(hvvr_gpu_view* v, const hvvr_gpu_scene* s, hipStream_t stream,
@@ -1310,16 +1879,16 @@ void launchTileListsBatch(const TileListArgs* all, const uint32_t* start, uint32
                           const LaunchShape& shape, hipStream_t stream) {
     tileListBatchKernel<<<units, 64, 0, stream>>>(all, start, viewCount, shape.xcdSwizzle);
     tileListQueueBatchKernel<TileListLarge>
-        <<<clampGroups(std::min(shape.largeGroups, uint32_t(kMaxLargeGroups)), units), 64, 0, stream>>>(
-            all + viewCount, viewCount);
+        <<<clampGroups(std::min(shape.largeGroups, uint32_t(kMaxLargeGroups)), units), 64 * TileListLarge::Waves, 0,
+           stream>>>(all + viewCount, viewCount);
     tileListQueueBatchKernel<TileListHuge>
-        <<<clampGroups(std::min(shape.hugeGroups, uint32_t(kMaxHugeGroups)), units), 64, 0, stream>>>(
-            all + 2 * viewCount, viewCount);
+        <<<clampGroups(std::min(shape.hugeGroups, uint32_t(kMaxHugeGroups)), units), 64 * TileListHuge::Waves, 0,
+           stream>>>(all + 2 * viewCount, viewCount);
     tileListQueueBatchKernel<TileListGiant>
-        <<<clampGroups(std::min(shape.giantGroups, uint32_t(kMaxGiantGroups)), units), 64, 0, stream>>>(
-            all + 3 * viewCount, viewCount);
-    tileListQueueBatchKernel<TileListColossal>
-        <<<clampGroups(uint32_t(kMaxColossalGroups), units), 64, 0, stream>>>(all + 4 * viewCount, viewCount);
+        <<<clampGroups(std::min(shape.giantGroups, uint32_t(kMaxGiantGroups)), units), 64 * TileListGiant::Waves, 0,
+           stream>>>(all + 3 * viewCount, viewCount);
+    tileSerialBatchKernel<<<clampGroups(uint32_t(kMaxColossalGroups), units), 64, 0, stream>>>(all + 4 * viewCount,
+                                                                                              viewCount);
 }
 
 void launchTileWalkBatch(const TileWalkArgs* all, uint32_t viewCount, uint32_t maxTiles, const LaunchShape& shape,

@@ -211,13 +211,12 @@ int hvvr_gpu_batch_synchronize(hvvr_gpu_batch* batch, float* gpuMs);
 int hvvr_gpu_batch_autotune(hvvr_gpu_batch* batch, hvvr_gpu_scene* scene, const float* cameraToWorld,
                             uint32_t framesPerTrial, hvvr_gpu_launch_shape* best, float* bestMs);
 
-/* Tile traversal keeps its distance-sorted stack in registers, up to `entries` (1..64,
- * default 64; it holds only nodes that still have work). Tiles that need more (or more
- * than 768 visited nodes, or that meet a NaN distance) go to larger configurations (2048,
- * 4608 and 10240 nodes; 256, 512 and 1024 stack entries, scaled down with a limit below
- * 64) and what none holds to a walk with the reference's full-depth stack (4096 entries,
- * TileFrame::stackSize, traverse_avx.h:281) in LDS. The result is the same either way;
- * the limit only moves work between the paths. */
+/* Tile traversal starts from its block's stack, up to `entries` of it (1..64, default 64).
+ * Tiles whose block stack holds more go to a walk with the reference's full-depth stack
+ * (4096 entries, TileFrame::stackSize, traverse_avx.h:281) in LDS; so do tiles that visit
+ * more nodes than the largest configuration holds (680, 2016, 4608, 9984 and, with a
+ * stack of 1024 entries, 20480) or that meet a NaN distance. The result is the same
+ * either way; the limit only moves work between the paths. */
 int hvvr_gpu_view_set_traversal_stack_limit(hvvr_gpu_view* view, uint32_t entries);
 /* 32 (default): FP32 shading, the oracle's arithmetic. 16: the GGX colour terms of each
  * light in packed FP16 (the scalar D / visibility / Fresnel weights and the radiance sum
@@ -341,7 +340,8 @@ typedef struct {
     uint64_t survivorPairs;    /* sum over tiles of 128 x triangles surviving the tile culls */
     uint32_t occupiedTiles;
     uint32_t tileCount;
-    uint32_t maxTileStack;     /* deepest tile traversal stack seen */
+    uint32_t maxTileStack;     /* deepest tile traversal stack seen: a serial walk's, or the block
+                                  stack a tile's traversal started from */
     uint32_t overflow;         /* nonzero if a budget overflowed */
     uint64_t nodeVisits;       /* BVH nodes tested by the tile traversal (4 child boxes each) */
     uint32_t largeTiles;       /* tiles the standard LDS configuration passed to the large one */

@@ -1,0 +1,72 @@
+"""The tile lists' order where the sort of the emitting records can go wrong, against the
+oracle's walk (traverse_avx.h:412-527): exact ties of distance keys between and within
+subtrees (boxes on a regular grid, whose faces share coordinates), cameras whose tiles and
+blocks have different distance axes (a yaw of 45 degrees, a pitch), tiles of one triangle up
+to tiles that need the large, huge and giant configurations."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid_scene(H, nx, ny, nz, size):
+    corner = np.array([[i & 1, (i >> 1) & 1, i >> 2] for i in range(8)], np.float64) - 0.5
+    quads = np.array([(1, 3, 7, 5), (0, 4, 6, 2), (2, 6, 7, 3), (0, 1, 5, 4), (4, 5, 7, 6), (0, 2, 3, 1)])
+    box = np.concatenate([quads[:, [0, 1, 2]], quads[:, [0, 2, 3]]])
+    centre = np.stack(np.meshgrid(np.arange(nx), np.arange(ny), np.arange(nz), indexing="ij"), -1).reshape(-1, 1, 3)
+    pos = (corner * size + centre).reshape(-1, 3)
+    tri = (box[None] + 8 * np.arange(len(centre))[:, None, None]).reshape(-1, 3)
+    v = np.zeros(len(pos), H.DTYPES["vertex"])
+    v["pos"] = pos
+    v["normal"][:, 1] = np.float16(1).view(np.uint16)
+    m = np.zeros(1, H.DTYPES["material"])
+    m["diffuse"] = (0.5, 0.5, 0.5, 1)
+    m["textureIDsAndShadingModel"] = 1 | (0xFFFF << 16) | (0xFFFF << 32) | (0xFFFF << 48)
+    return H.HostScene.from_meshes([(v, tri.astype(np.uint32), np.zeros(len(tri), np.uint32), None)], m)
+
+
+def _camera(H, pos, yaw, pitch):
+    a, b = np.radians(yaw) / 2, np.radians(pitch) / 2
+    cy, sy, cp, sp = np.cos(a), np.sin(a), np.cos(b), np.sin(b)
+    return H.transform_matrix(np.array(pos), np.array([cy * sp, sy * cp, -sy * sp, cy * cp]))
+
+
+def _check(H, O, ctx, scene, view, m):
+    ref = O.render_view(scene, view, 1, camera_to_world=m, with_colors=False)
+    total = int(ref["counts"].sum())
+    assert total > 0
+    gs = H.GpuScene(ctx, scene)
+    gv = H.GpuView(ctx, view, 1)
+    gv.reserve_lists(total)
+    for _ in range(2):  # the second frame follows the per-tile hints
+        gv.render(gs, m)
+        counts, lists = gv.read_tile_lists()
+        assert np.array_equal(counts, ref["counts"]), "tile list lengths differ"
+        assert np.array_equal(lists, ref["lists"]), "tile list contents/order differ"
+    st = gv.stats()
+    gv.close()
+    gs.close()
+    return st
+
+
+@pytest.mark.parametrize("yaw,pitch", [(0, 0), (45, 0), (30, 20), (10, -35)])
+@pytest.mark.parametrize("grid", [(1, 1, 1, 0.6), (16, 8, 16, 0.5), (20, 20, 20, 0.3), (64, 2, 64, 0.9)])
+def test_ties_on_a_grid(H, O, ctx, grid, yaw, pitch):
+    nx, ny, nz, size = grid
+    scene = _grid_scene(H, nx, ny, nz, size)
+    view = H.HostView(H.VIEW_PRESET_ROOM_EYE, 0, 320, 320)
+    m = _camera(H, (nx / 2 - 0.2, ny / 2 + 0.3, nz + 2.0), yaw, pitch)
+    st = _check(H, O, ctx, scene, view, m)
+    assert st.colossalTiles == 0 and st.walkTiles == 0
+
+
+@pytest.mark.parametrize("yaw,pitch", [(0, 0), (45, 10)])
+@pytest.mark.parametrize("meshes,size", [(64, 48), (391, 129), (1024, 96), (4096, 160), (8192, 128)])
+def test_room_tiles_of_every_configuration(H, O, ctx, meshes, size, yaw, pitch):
+    # 64 meshes: a few records per tile; 8,192 at 128x128: up to the giant configuration
+    scene = H.HostScene(H.SCENE_ROOM, 1, meshes)
+    view = H.HostView(H.VIEW_PRESET_ROOM_EYE, 1, size, size)
+    st = _check(H, O, ctx, scene, view, _camera(H, (15.0, 7.5, 27.0), yaw, pitch))
+    if meshes == 8192:
+        assert st.hugeTiles > 0 and st.giantTiles > 0
