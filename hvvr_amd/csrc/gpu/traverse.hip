@@ -287,12 +287,15 @@ __global__ __launch_bounds__(64) void blockTraverseBatchKernel(const BlockTraver
 // configuration replays the walk with one wave (tileSerialBody), and what that cannot hold
 // goes to the wave-per-tile walk with its stack in LDS.
 // ---------------------------------------------------------------------------------
-// Record meta: first child record (bits 0..19), child mask (20..23), leaf mask (24..27),
-// stack-entry leaf mask (28..31).
+// Record meta: first child record (bits 0..19; in the standard configuration bits 0..9, rp
+// in bits 10..19), child mask (20..23), leaf mask (24..27), stack-entry leaf mask (28..31).
 __device__ inline uint32_t metaMask(uint32_t m) { return (m >> 20) & 0xfu; }
 __device__ inline uint32_t metaLeaf(uint32_t m) { return (m >> 24) & 0xfu; }
 __device__ inline uint32_t metaEntry(uint32_t m) { return m >> 28; }
-__device__ inline uint32_t metaFirst(uint32_t m) { return m & 0xfffffu; }
+template <class Cfg>
+__device__ inline uint32_t metaFirst(uint32_t m) {
+    return m & (Cfg::Packed ? 0x3ffu : 0xfffffu);
+}
 __device__ inline uint32_t packMeta(uint32_t first, uint32_t mask, uint32_t leaf, uint32_t entry) {
     return first | (mask << 20) | (leaf << 24) | (entry << 28);
 }
@@ -301,24 +304,25 @@ __device__ inline uint32_t packMeta(uint32_t first, uint32_t mask, uint32_t leaf
 __device__ inline uint32_t metaInner(uint32_t m) { return metaEntry(m) == 0u ? metaMask(m) & ~metaLeaf(m) : 0u; }
 __device__ inline uint32_t metaEmits(uint32_t m) { return metaMask(m) & metaLeaf(m); }
 
-// 16 bytes of LDS per record: 680 records of one wave let a CU hold 14 tiles; 2016 records
-// five workgroups (20 waves), 4608 two (16 waves), 9984 one (16 waves).
+// 14 bytes of LDS per record in the standard configuration, 16 in the others: a CU holds 19
+// of the first's single waves, five workgroups of the large configuration (20 waves), two
+// of the huge one (16) and one of the giant one (16).
 struct TileListSmall {
-    enum : uint32_t { RecCap = 680, Waves = 1, Slots = 2, Level = 0 };
+    enum : uint32_t { RecCap = 576, Waves = 1, Slots = 2, Level = 0, Occupancy = 5, Packed = 1, Chunks = 32 };
 };
 struct TileListLarge {
-    enum : uint32_t { RecCap = 2016, Waves = 4, Slots = 2, Level = 1, Occupancy = 5 };
+    enum : uint32_t { RecCap = 2016, Waves = 4, Slots = 2, Level = 1, Occupancy = 5, Packed = 0, Chunks = 64 };
 };
 struct TileListHuge {
-    enum : uint32_t { RecCap = 4608, Waves = 8, Slots = 2, Level = 2, Occupancy = 4 };
+    enum : uint32_t { RecCap = 4608, Waves = 8, Slots = 2, Level = 2, Occupancy = 4, Packed = 0, Chunks = 64 };
 };
 struct TileListGiant {
-    enum : uint32_t { RecCap = 9984, Waves = 16, Slots = 2, Level = 3, Occupancy = 4 };
+    enum : uint32_t { RecCap = 9984, Waves = 16, Slots = 2, Level = 3, Occupancy = 4, Packed = 0, Chunks = 64 };
 };
 // the serial walk's: keys and metas in LDS (all 160 KB), node indices and emission order in
 // global scratch, a sixteen-register stack
 struct TileListColossal {
-    enum : uint32_t { RecCap = 20480, StackCap = REG_STACK16_CAP, Level = 4, Slots = 4 };
+    enum : uint32_t { RecCap = 20480, StackCap = REG_STACK16_CAP, Level = 4, Slots = 4, Packed = 0 };
     using Stack = RegStack16;
 };
 
@@ -329,34 +333,81 @@ constexpr uint32_t recScratchWords() {
 }
 
 enum : uint32_t {
-    kMaxTileChunks = 64,   // chunks of the records' up and down passes
-    kNoRecord = 0xffffu,   // the rp of a block-stack entry's tree
     kOldest = 0xffffffffu, // ~W[rp] of such a tree: older than any pushed entry
     kUncovered = 0xffffffc0u // merged families: the entries' own place, by position below it
 };
 
+// per record, besides meta and node: the float bits of W, rp, and the number of live records
+// in its subtree, then D
+template <class Cfg, bool Packed = bool(Cfg::Packed)>
+struct TileRecords {
+    uint32_t key[Cfg::RecCap];
+    uint16_t number[Cfg::RecCap]; // (rp is in the meta)
+};
+template <class Cfg>
+struct TileRecords<Cfg, false> {
+    uint32_t key[Cfg::RecCap];
+    uint32_t aux[Cfg::RecCap]; // rp << 16 | number
+};
+
 // An emitting record as a sort element: W and ~W[rp] as order-preserving integers, D[rp]
-// (descending) << 16 | D, and rp[rp] << 16 | record.
+// (descending) << 16 | D, and rp[rp] << 16 | record. The elements take the place of the
+// records' keys and numbers.
 template <class Cfg>
 struct TileListLds {
-    enum : uint32_t { ElemCap = Cfg::RecCap / 2 };
-    uint32_t meta[Cfg::RecCap]; // packMeta; after the passes, low bits: the emitting records' list
-    uint32_t node[Cfg::RecCap];
-    union {
-        struct {
-            uint32_t key[Cfg::RecCap]; // float bits of W
-            uint32_t aux[Cfg::RecCap]; // rp << 16 | live records in the subtree, then D
-        };
-        uint4 elem[ElemCap];
+    enum : uint32_t {
+        ElemCap = uint32_t(sizeof(TileRecords<Cfg>) / sizeof(uint4)),
+        NoRecord = Cfg::Packed ? 0x3ffu : 0xffffu // the rp of a block-stack entry's tree
     };
+    union {
+        uint4 elem[ElemCap];
+        TileRecords<Cfg> rec;
+    };
+    uint32_t meta[Cfg::RecCap]; // after the passes, the low bits: the emitting records' list
+    uint32_t node[Cfg::RecCap];
     uint32_t appended[3]; // children appended in a step (several waves), in turn
     uint32_t bad;         // a NaN or infinite key; later, an order the sort does not decide
     uint32_t emitters;
     uint32_t waveTotals[Cfg::Waves];
     uint32_t listStart[2]; // 64-bit list start, and whether the list fits
     uint32_t listFits;
-    uint16_t chunk[kMaxTileChunks + 1]; // first record of each chunk
-    uint16_t familyD[64];               // first D of each block-stack entry's family
+    uint16_t chunk[Cfg::Chunks + 1]; // first record of each chunk of the up and down passes
+    uint16_t familyD[64];            // first D of each block-stack entry's family
+
+    __device__ uint32_t rp(uint32_t r) const {
+        if constexpr (Cfg::Packed)
+            return (meta[r] >> 10) & 0x3ffu;
+        else
+            return rec.aux[r] >> 16;
+    }
+    __device__ uint32_t number(uint32_t r) const {
+        if constexpr (Cfg::Packed)
+            return rec.number[r];
+        else
+            return rec.aux[r] & 0xffffu;
+    }
+    // (the low half alone: the rp stays)
+    __device__ void setNumber(uint32_t r, uint32_t n) {
+        if constexpr (Cfg::Packed)
+            rec.number[r] = uint16_t(n);
+        else
+            reinterpret_cast<uint16_t*>(&rec.aux[r])[0] = uint16_t(n);
+    }
+    // a new record, its subtree not counted yet
+    __device__ void create(uint32_t r, uint32_t nodeIndex, float w, uint32_t rpr, uint32_t entry) {
+        node[r] = nodeIndex;
+        rec.key[r] = fbits(w);
+        if constexpr (Cfg::Packed) {
+            meta[r] = packMeta(rpr << 10, 0u, 0u, entry);
+            rec.number[r] = 0;
+        } else {
+            meta[r] = packMeta(0u, 0u, 0u, entry);
+            rec.aux[r] = rpr << 16;
+        }
+    }
+    __device__ void setMeta(uint32_t r, uint32_t first, uint32_t mask, uint32_t leaf, uint32_t entry, uint32_t rpr) {
+        meta[r] = packMeta(Cfg::Packed ? first | (rpr << 10) : first, mask, leaf, entry);
+    }
 };
 
 // every wave's LDS accesses before it are complete and seen by the others after it
@@ -509,6 +560,24 @@ __device__ inline bool elemLess(const uint4& x, const uint4& y) {
 template <class Cfg>
 __device__ inline void sortElements(TileListLds<Cfg>& sh, uint32_t n, uint32_t tid) {
     constexpr uint32_t T = 64 * Cfg::Waves;
+    if (Cfg::Waves == 1 && n <= 64u) {
+        // one element per lane, its rank the number of elements before it (about 8
+        // instructions each, where the network takes 21 stages of four LDS accesses)
+        waveLdsSync();
+        const uint4 e = sh.elem[tid < n ? tid : 0u];
+        const uint64_t hi = (uint64_t(e.x) << 32) | e.y;
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < n; j++) {
+            const uint64_t other = (uint64_t(readLane(e.x, j)) << 32) | readLane(e.y, j);
+            const uint32_t z = readLane(e.z, j);
+            rank += (other < hi) | ((other == hi) & (z < e.z)) ? 1u : 0u;
+        }
+        waveLdsSync();
+        if (tid < n)
+            sh.elem[rank] = e;
+        waveLdsSync();
+        return;
+    }
     uint32_t P = 2;
     while (P < n)
         P <<= 1;
@@ -567,21 +636,22 @@ template <class Cfg>
 __device__ bool visitedBefore(const TileListLds<Cfg>& sh, uint32_t x, uint32_t y, bool families, uint32_t n0,
                               const StackEntry* bs) {
     for (;;) {
-        const uint32_t ax = sh.aux[x], ay = sh.aux[y];
-        const uint32_t wx = orderedKey(bitsf(sh.key[x])), wy = orderedKey(bitsf(sh.key[y]));
+        const uint32_t wx = orderedKey(bitsf(sh.rec.key[x])), wy = orderedKey(bitsf(sh.rec.key[y]));
+        const uint32_t dx = sh.number(x), dy = sh.number(y), px = sh.rp(x), py = sh.rp(y);
+        constexpr uint32_t none = TileListLds<Cfg>::NoRecord;
         uint32_t fx = 0, fy = 0;
         if (families) {
-            fx = familyOf(sh, n0, ax & 0xffffu);
-            fy = familyOf(sh, n0, ay & 0xffffu);
+            fx = familyOf(sh, n0, dx);
+            fy = familyOf(sh, n0, dy);
         }
         if (fx == fy) {
             if (wx != wy)
                 return wx < wy;
-            if ((ax >> 16) == (ay >> 16))
-                return (ax & 0xffffu) < (ay & 0xffffu);
-            if ((ax >> 16) == kNoRecord)
+            if (px == py)
+                return dx < dy;
+            if (px == none)
                 return false;
-            if ((ay >> 16) == kNoRecord)
+            if (py == none)
                 return true;
         } else {
             const uint32_t kx = orderedKey(bs[fx].tMin), ky = orderedKey(bs[fy].tMin);
@@ -591,8 +661,8 @@ __device__ bool visitedBefore(const TileListLds<Cfg>& sh, uint32_t x, uint32_t y
             if (!(wx > kx) || !(wy > ky))
                 return (wx > kx) || (!(wy > ky) && fx > fy);
         }
-        x = ay >> 16; // the one whose tree was pushed later comes first
-        y = ax >> 16;
+        x = py; // the one whose tree was pushed later comes first
+        y = px;
     }
 }
 
@@ -602,7 +672,7 @@ template <class Cfg>
 __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, uint32_t tile, uint32_t tid,
                                    bool rank) {
     constexpr uint32_t Waves = Cfg::Waves, T = 64 * Waves, RecCap = Cfg::RecCap;
-    constexpr uint32_t ElemCap = TileListLds<Cfg>::ElemCap;
+    constexpr uint32_t ElemCap = TileListLds<Cfg>::ElemCap, NoRecord = TileListLds<Cfg>::NoRecord;
     const uint32_t lane = tid & 63u, wave = Waves == 1 ? 0u : uniform(tid >> 6);
     const BVHNode* __restrict__ nodes = g.nodes;
     const uint32_t block = tile / TILES_PER_BLOCK;
@@ -636,10 +706,7 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
         const float t = lane < n0 ? bs[lane].tMin : 0.0f;
         if (lane < n0) {
             const uint32_t m = bs[lane].nodeMask;
-            sh.node[lane] = m & STACK_NODE_MASK;
-            sh.key[lane] = fbits(families ? -INFINITY : t);
-            sh.meta[lane] = packMeta(0u, 0u, 0u, m >> 28);
-            sh.aux[lane] = kNoRecord << 16;
+            sh.create(lane, m & STACK_NODE_MASK, families ? -INFINITY : t, NoRecord, m >> 28);
         }
         const float above = __shfl_down(t, 1);
         bad = !(fabsf(t) <= FLT_MAX) || (lane + 1u < n0 && t < above);
@@ -662,7 +729,7 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
             const uint32_t end = head + 16 * S * Waves < nrec ? head + 16 * S * Waves : nrec;
             // a chunk: up to T records whose children all lie past it
             if (end > chunkEnd) {
-                if (chunks == kMaxTileChunks)
+                if (chunks == uint32_t(Cfg::Chunks))
                     return give(TileResult::TooBig);
                 if (tid == 0)
                     sh.chunk[chunks] = uint16_t(head);
@@ -681,8 +748,8 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
                 if (valid[k]) {
                     nodeR[k] = sh.node[recI[k]];
                     entryR[k] = metaEntry(sh.meta[recI[k]]);
-                    wR[k] = bitsf(sh.key[recI[k]]);
-                    rpR[k] = sh.aux[recI[k]] >> 16;
+                    wR[k] = bitsf(sh.rec.key[recI[k]]);
+                    rpR[k] = sh.rp(recI[k]);
                 }
             }
             ChildBox X[S];
@@ -724,14 +791,11 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
                 const bool only = __builtin_popcount(uint32_t(bi[k] >> (4 * s)) & 0xfu) == 1;
                 if (inner[k] && slot < RecCap) {
                     const float w = only ? wR[k] : X[k].key;
-                    sh.node[slot] = nodeR[k] + X[k].childOffset;
-                    sh.key[slot] = fbits(w);
-                    sh.meta[slot] = 0u;
-                    sh.aux[slot] = (w == wR[k] ? rpR[k] : recI[k]) << 16;
+                    sh.create(slot, nodeR[k] + X[k].childOffset, w, w == wR[k] ? rpR[k] : recI[k], 0u);
                 }
                 if (valid[k] && c == 0) {
                     const uint32_t first = base + uint32_t(__builtin_popcountll(bi[k] & groupBelow));
-                    sh.meta[recI[k]] = packMeta(first, maskK, X[k].leafMask, entryR[k]);
+                    sh.setMeta(recI[k], first, maskK, X[k].leafMask, entryR[k], rpR[k]);
                 }
                 base += uint32_t(__builtin_popcountll(bi[k]));
                 // (a key below its parent's W has no place in the order; boxes that nest
@@ -770,25 +834,25 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
     for (uint32_t k = chunks; k-- > 0;) {
         const uint32_t r = sh.chunk[k] + tid;
         if (r < sh.chunk[k + 1]) {
-            const uint32_t m = sh.meta[r], first = metaFirst(m);
+            const uint32_t m = sh.meta[r], first = metaFirst<Cfg>(m);
             const uint32_t n = uint32_t(__builtin_popcount(metaInner(m)));
             uint32_t live = 0;
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++)
                 if (j < n)
-                    live += sh.aux[first + j] & 0xffffu;
+                    live += sh.number(first + j);
             if (live != 0u || metaEmits(m) != 0u)
-                sh.aux[r] |= live + 1u;
+                sh.setNumber(r, live + 1u);
         }
         tileSync<Waves>();
     }
     // Down: D, from the block-stack entries, the highest position first.
     if (wave == 0) {
         const uint32_t q = n0 - 1u - lane;
-        const uint32_t a = lane < n0 ? sh.aux[q] : 0u, live = a & 0xffffu;
+        const uint32_t live = lane < n0 ? sh.number(q) : 0u;
         const uint32_t d = 1u + waveInclusiveScan(live) - live;
         if (lane < n0) {
-            sh.aux[q] = (a & 0xffff0000u) | d;
+            sh.setNumber(q, d);
             sh.familyD[q] = uint16_t(d);
         }
     }
@@ -799,18 +863,18 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
         const bool mine = r < sh.chunk[k + 1];
         bool emits = false;
         if (mine) {
-            const uint32_t m = sh.meta[r], first = metaFirst(m);
+            const uint32_t m = sh.meta[r], first = metaFirst<Cfg>(m);
             const uint32_t n = uint32_t(__builtin_popcount(metaInner(m)));
             emits = metaEmits(m) != 0u;
-            uint32_t d = (sh.aux[r] & 0xffffu) + 1u, a[4];
+            uint32_t d = sh.number(r) + 1u, live[4];
 #pragma unroll
             for (uint32_t j = 0; j < 4; j++)
-                a[j] = j < n ? sh.aux[first + j] : 0u;
+                live[j] = j < n ? sh.number(first + j) : 0u;
 #pragma unroll
             for (uint32_t j = 4; j-- > 0;)
                 if (j < n) {
-                    sh.aux[first + j] = (a[j] & 0xffff0000u) | d;
-                    d += a[j] & 0xffffu;
+                    sh.setNumber(first + j, d);
+                    d += live[j];
                 }
         }
         // the emitting records' list, in any order, in the low bits of the metas of
@@ -822,7 +886,7 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
         at = readLane(at, 0) + lanesBelow(be);
         tileSync<Waves>();
         if (emits)
-            sh.meta[at] = (sh.meta[at] & 0xfff00000u) | r;
+            sh.meta[at] = (sh.meta[at] & ~(Cfg::Packed ? 0x3ffu : 0xfffffu)) | r;
     }
     tileSync<Waves>();
     const uint32_t nEmit = uniform(sh.emitters);
@@ -836,9 +900,9 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
         for (uint32_t k = 0; k < K; k++) {
             at[k] = rec[k] = 0;
             if (k * T + tid < nEmit) {
-                rec[k] = metaFirst(sh.meta[k * T + tid]);
+                rec[k] = metaFirst<Cfg>(sh.meta[k * T + tid]);
                 for (uint32_t i = 0; i < nEmit; i++)
-                    at[k] += visitedBefore(sh, metaFirst(sh.meta[i]), rec[k], families, n0, bs) ? 1u : 0u;
+                    at[k] += visitedBefore(sh, metaFirst<Cfg>(sh.meta[i]), rec[k], families, n0, bs) ? 1u : 0u;
             }
         }
         tileSync<Waves>();
@@ -853,17 +917,16 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
         for (uint32_t k = 0; k < K; k++) {
             const uint32_t i = k * T + tid;
             if (i < nEmit) {
-                const uint32_t r = metaFirst(sh.meta[i]), a = sh.aux[r], rp = a >> 16;
-                e[k].x = orderedKey(bitsf(sh.key[r]));
-                if (rp == kNoRecord) {
+                const uint32_t r = metaFirst<Cfg>(sh.meta[i]), rp = sh.rp(r);
+                e[k].x = orderedKey(bitsf(sh.rec.key[r]));
+                if (rp == NoRecord) {
                     e[k].y = kOldest;
-                    e[k].z = 0xffff0000u | (a & 0xffffu);
+                    e[k].z = 0xffff0000u | sh.number(r);
                     e[k].w = 0xffff0000u | r;
                 } else {
-                    const uint32_t p = sh.aux[rp];
-                    e[k].y = ~orderedKey(bitsf(sh.key[rp]));
-                    e[k].z = (~p << 16) | (a & 0xffffu);
-                    e[k].w = (p & 0xffff0000u) | r;
+                    e[k].y = ~orderedKey(bitsf(sh.rec.key[rp]));
+                    e[k].z = (~sh.number(rp) << 16) | sh.number(r);
+                    e[k].w = (sh.rp(rp) << 16) | r;
                 }
             }
         }
@@ -1013,14 +1076,15 @@ __device__ inline bool followHint(const TileListArgs& g, uint32_t level, uint32_
 }
 
 // every tile, standard configuration
-__global__ __launch_bounds__(64) void tileListKernel(TileListArgs g) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TileListSmall::Occupancy)))
+void tileListKernel(TileListArgs g) {
     __shared__ TileListLds<TileListSmall> sh;
     tileListOne(g, sh, blockIdx.x, threadIdx.x);
 }
 
-__global__ __launch_bounds__(64) void tileListBatchKernel(const TileListArgs* __restrict__ all,
-                                                          const uint32_t* __restrict__ start, uint32_t n,
-                                                          uint32_t swizzle) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TileListSmall::Occupancy)))
+void tileListBatchKernel(const TileListArgs* __restrict__ all, const uint32_t* __restrict__ start, uint32_t n,
+                         uint32_t swizzle) {
     __shared__ TileListLds<TileListSmall> sh;
     const uint32_t unit = xcdUnit(blockIdx.x, gridDim.x, swizzle);
     const uint32_t v = batchView(start, n, unit);
@@ -1202,7 +1266,7 @@ __device__ bool tileSerialBody(const TileListArgs& g, TileSerialLds& sh, uint32_
             const uint32_t meta = valid ? sh.recMeta[r] : 0u;
             const uint32_t mask = metaMask(meta), leaf = metaLeaf(meta);
             const uint32_t inner = metaEntry(meta) == 0u ? mask & ~leaf : 0u;
-            const uint32_t first = metaFirst(meta);
+            const uint32_t first = metaFirst<Cfg>(meta);
             const uint32_t nInner = uint32_t(__builtin_popcount(inner));
             // emitting records keep their mask; the others keep it while a child is live
             bool open = valid && mask != 0u && (mask & leaf) == 0u;
@@ -1280,7 +1344,7 @@ __device__ bool tileSerialBody(const TileListArgs& g, TileSerialLds& sh, uint32_
             if (inner != 0u) {
                 // the hit children's records, contiguous from `first` in child order; lanes
                 // past them read an in-range record and are masked off
-                const uint32_t first = metaFirst(curMeta);
+                const uint32_t first = metaFirst<Cfg>(curMeta);
                 const uint32_t nChildren = uint32_t(__builtin_popcount(inner));
                 const uint32_t r = first + lane < uint32_t(Cfg::RecCap) ? first + lane : uint32_t(Cfg::RecCap) - 1u;
                 const uint32_t childKey = sh.recKey[r];
