@@ -553,13 +553,41 @@ __device__ inline bool elemLess(const uint4& x, const uint4& y) {
     return x.x < y.x || (x.x == y.x && (x.y < y.y || (x.y == y.y && x.z < y.z)));
 }
 
-// Sorts sh.elem[0, n) ascending (a bitonic network whose comparators all point up, so the
-// missing elements past n need no padding). Comparator i of a stage of stride up to 64
-// touches the aligned 128 elements of its 64-comparator block, which one wave holds: such
-// stages need no workgroup barrier.
+// The comparators of a bitonic network over n elements: exchange(lo, hi) puts the lesser of
+// two elements at lo. All comparators point up, so the missing elements past n need no
+// padding. Comparator i of a stage of stride up to 64 touches the aligned 128 elements of
+// its 64-comparator block, which one wave holds: such stages need no workgroup barrier.
+template <uint32_t Waves, class Exchange>
+__device__ inline void sortNetwork(uint32_t n, uint32_t tid, Exchange exchange) {
+    constexpr uint32_t T = 64 * Waves;
+    uint32_t P = 2;
+    while (P < n)
+        P <<= 1;
+    tileSync<Waves>();
+    for (uint32_t size = 2; size <= P; size <<= 1) {
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            if (Waves > 1 && stride > 64u)
+                __syncthreads();
+            const bool flip = stride == size >> 1;
+#pragma unroll 1
+            for (uint32_t i = tid; i < P / 2; i += T) {
+                const uint32_t off = i & (stride - 1u), base = (i - off) << 1;
+                const uint32_t hi = flip ? base + size - 1u - off : base + off + stride;
+                if (hi < n)
+                    exchange(base + off, hi);
+            }
+            if (Waves > 1 && stride > 64u)
+                __syncthreads();
+            else
+                waveLdsSync();
+        }
+    }
+    tileSync<Waves>();
+}
+
+// sorts sh.elem[0, n) ascending
 template <class Cfg>
 __device__ inline void sortElements(TileListLds<Cfg>& sh, uint32_t n, uint32_t tid) {
-    constexpr uint32_t T = 64 * Cfg::Waves;
     if (Cfg::Waves == 1 && n <= 64u) {
         // one element per lane, its rank the number of elements before it (about 8
         // instructions each, where the network takes 21 stages of four LDS accesses)
@@ -578,36 +606,13 @@ __device__ inline void sortElements(TileListLds<Cfg>& sh, uint32_t n, uint32_t t
         waveLdsSync();
         return;
     }
-    uint32_t P = 2;
-    while (P < n)
-        P <<= 1;
-    auto exchange = [&](uint32_t lo, uint32_t hi) {
-        if (hi < n) {
-            const uint4 a = sh.elem[lo], b = sh.elem[hi];
-            if (elemLess(b, a)) {
-                sh.elem[lo] = b;
-                sh.elem[hi] = a;
-            }
+    sortNetwork<Cfg::Waves>(n, tid, [&](uint32_t lo, uint32_t hi) {
+        const uint4 a = sh.elem[lo], b = sh.elem[hi];
+        if (elemLess(b, a)) {
+            sh.elem[lo] = b;
+            sh.elem[hi] = a;
         }
-    };
-    tileSync<Cfg::Waves>();
-    for (uint32_t size = 2; size <= P; size <<= 1) {
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            if (Cfg::Waves > 1 && stride > 64u)
-                __syncthreads();
-            const bool flip = stride == size >> 1;
-#pragma unroll 1
-            for (uint32_t i = tid; i < P / 2; i += T) {
-                const uint32_t off = i & (stride - 1u), base = (i - off) << 1;
-                exchange(base + off, flip ? base + size - 1u - off : base + off + stride);
-            }
-            if (Cfg::Waves > 1 && stride > 64u)
-                __syncthreads();
-            else
-                waveLdsSync();
-        }
-    }
-    tileSync<Cfg::Waves>();
+    });
 }
 
 enum class TileResult : uint32_t { Done, TooBig, Irregular, Undecided };
@@ -895,23 +900,79 @@ __device__ TileResult tileListBody(const TileListArgs& g, TileListLds<Cfg>& sh, 
     constexpr uint32_t K = (ElemCap + T - 1) / T; // elements per thread
     bad = false;
     if (rank) {
-        uint32_t at[K], rec[K];
+        // the key a comparison starts with (E where families merge, else W)
+        auto firstKey = [&](uint32_t r) {
+            const uint32_t w = orderedKey(bitsf(sh.rec.key[r]));
+            if (!families)
+                return w;
+            const uint32_t key = orderedKey(bs[familyOf(sh, n0, sh.number(r))].tMin);
+            return w > key ? w : key;
+        };
+        uint32_t key[K], rec[K];
 #pragma unroll
         for (uint32_t k = 0; k < K; k++) {
-            at[k] = rec[k] = 0;
+            key[k] = rec[k] = 0;
             if (k * T + tid < nEmit) {
                 rec[k] = metaFirst<Cfg>(sh.meta[k * T + tid]);
-                for (uint32_t i = 0; i < nEmit; i++)
-                    at[k] += visitedBefore(sh, metaFirst<Cfg>(sh.meta[i]), rec[k], families, n0, bs) ? 1u : 0u;
+                key[k] = firstKey(rec[k]);
             }
         }
-        tileSync<Waves>();
+        if constexpr (Cfg::Packed) {
+            // few records (and their rps are in the metas): each one's rank by counting
+            uint32_t at[K];
 #pragma unroll
-        for (uint32_t k = 0; k < K; k++)
-            if (k * T + tid < nEmit)
-                sh.elem[at[k]].w = rec[k];
+            for (uint32_t k = 0; k < K; k++) {
+                at[k] = 0;
+                for (uint32_t i = 0; i < nEmit; i++) {
+                    const uint32_t r = metaFirst<Cfg>(sh.meta[i]), other = firstKey(r);
+                    if (k * T + tid < nEmit)
+                        at[k] += (other == key[k] ? visitedBefore(sh, r, rec[k], families, n0, bs) : other < key[k])
+                                     ? 1u
+                                     : 0u;
+                }
+            }
+            tileSync<Waves>();
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++)
+                if (k * T + tid < nEmit)
+                    sh.elem[at[k]].w = rec[k];
+        } else {
+            // (key, record, emitting leaves) pairs in place of the metas, sorted with the
+            // full comparison where keys tie; then the leaves return to the metas
+            uint2* pair = reinterpret_cast<uint2*>(sh.meta);
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++)
+                rec[k] |= k * T + tid < nEmit ? metaEmits(sh.meta[rec[k]]) << 16 : 0u;
+            tileSync<Waves>();
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++)
+                if (k * T + tid < nEmit)
+                    pair[k * T + tid] = make_uint2(key[k], rec[k]);
+            sortNetwork<Waves>(nEmit, tid, [&](uint32_t lo, uint32_t hi) {
+                const uint2 a = pair[lo], b = pair[hi];
+                const bool swap = a.x == b.x
+                                      ? visitedBefore(sh, b.y & 0xffffu, a.y & 0xffffu, families, n0, bs)
+                                      : b.x < a.x;
+                if (swap) {
+                    pair[lo] = b;
+                    pair[hi] = a;
+                }
+            });
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++)
+                if (k * T + tid < nEmit)
+                    rec[k] = pair[k * T + tid].y;
+            tileSync<Waves>();
+#pragma unroll
+            for (uint32_t k = 0; k < K; k++)
+                if (k * T + tid < nEmit) {
+                    const uint32_t r = rec[k] & 0xffffu, leaves = rec[k] >> 16;
+                    sh.meta[r] = packMeta(0u, leaves, leaves, 0u);
+                    sh.elem[k * T + tid].w = r;
+                }
+        }
     } else {
-        // the elements take the place of the keys and aux words: through registers
+        // the elements take the place of the keys and numbers: through registers
         uint4 e[K];
 #pragma unroll
         for (uint32_t k = 0; k < K; k++) {

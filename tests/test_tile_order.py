@@ -61,6 +61,16 @@ def test_ties_on_a_grid(H, O, ctx, grid, yaw, pitch):
     assert st.colossalTiles == 0 and st.walkTiles == 0
 
 
+@pytest.mark.parametrize("yaw,pitch", [(0, 0), (30, 20)])
+@pytest.mark.parametrize("size", [24, 64])
+def test_ties_in_large_tiles(H, O, ctx, size, yaw, pitch):
+    # wide tiles over 30,720 equal boxes: ties in the configurations of several waves
+    scene = _grid_scene(H, 40, 24, 32, 0.3)
+    view = H.HostView(H.VIEW_PRESET_ROOM_EYE, 0, size, size)
+    st = _check(H, O, ctx, scene, view, _camera(H, (19.8, 12.3, 34.0), yaw, pitch))
+    assert st.largeTiles > 0
+
+
 @pytest.mark.parametrize("yaw,pitch", [(0, 0), (45, 10)])
 @pytest.mark.parametrize("meshes,size", [(64, 48), (391, 129), (1024, 96), (4096, 160), (8192, 128)])
 def test_room_tiles_of_every_configuration(H, O, ctx, meshes, size, yaw, pitch):
