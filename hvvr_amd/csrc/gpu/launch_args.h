@@ -98,6 +98,7 @@ struct IntersectArgs {
     vector4* hits;
     uint64_t listCapacity;
     matrix4x4 cameraToWorld;
+    vector2 offsetMax; // the largest |x| and |y| of the subsample offsets
     vector2 offsets[32];
     // depth of field: lens-position table [4][A][128], rank of each tile among the
     // tiles with a non-empty list (its table row is rank % 4), thin lens
