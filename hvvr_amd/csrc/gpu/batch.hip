@@ -158,9 +158,10 @@ int batchFail(const std::string& msg, int code = HVVR_GPU_ERR_INVALID) {
 
 // everything the launches depend on besides the per-frame arguments
 std::vector<uint64_t> frameSignature(const hvvr_gpu_batch* b, const hvvr_gpu_scene* s) {
-    // (whether the scene has textures picks the resolve variant a captured graph holds)
-    std::vector<uint64_t> sig = {uint64_t(uintptr_t(s)), uint64_t(s->textureCount > 0), uint64_t(b->refitEveryFrame),
-                                 b->shape.largeGroups,
+    // (whether the scene has textures picks the resolve variant a captured graph holds, its
+    // triangle count the intersect's)
+    std::vector<uint64_t> sig = {uint64_t(uintptr_t(s)), uint64_t(s->textureCount > 0), s->triangleCount,
+                                 uint64_t(b->refitEveryFrame), b->shape.largeGroups,
                                  b->shape.hugeGroups,    b->shape.giantGroups,          b->shape.walkGroups,
                                  b->shape.xcdSwizzle,    b->shape.streams};
     for (const hvvr_gpu_view* v : b->views) {
@@ -309,7 +310,7 @@ void fillArgs(Chain& c, const hvvr_gpu_scene* s, const matrix4x4* m) {
 }
 
 // one chain's work on its stream
-void enqueueChain(const hvvr_gpu_batch* b, Chain& c, bool tex) {
+void enqueueChain(const hvvr_gpu_batch* b, Chain& c, const hvvr_gpu_scene* s) {
     const uint32_t n = uint32_t(c.views.size());
     hipStream_t st = c.stream;
     uint8_t* d = c.devArgs.ptr;
@@ -326,8 +327,8 @@ void enqueueChain(const hvvr_gpu_batch* b, Chain& c, bool tex) {
     for (const Group& g : c.groups) {
         const uint32_t gn = uint32_t(g.members.size());
         launchIntersectBatch(int(g.msaaRate), reinterpret_cast<const IntersectArgs*>(d + g.intersectOff),
-                             u32(g.startOff), gn, g.units, b->shape, st);
-        launchResolveBatch(int(g.msaaRate), g.half, tex, reinterpret_cast<const ResolveArgs*>(d + g.resolveOff),
+                             u32(g.startOff), gn, g.units, s->triangleCount, b->shape, st);
+        launchResolveBatch(int(g.msaaRate), g.half, s->textureCount > 0, reinterpret_cast<const ResolveArgs*>(d + g.resolveOff),
                            u32(g.startOff), gn, g.units, b->shape, st);
     }
     if (!c.remapMembers.empty())
@@ -353,7 +354,7 @@ void enqueueFrame(hvvr_gpu_batch* b, hvvr_gpu_scene* s, bool graphs) {
         if (graphs)
             (void)hipGraphLaunch(b->execs[k], c.stream ? c.stream : b->stream);
         else
-            enqueueChain(b, c, s->textureCount > 0);
+            enqueueChain(b, c, s);
     }
     for (size_t k = 1; k < b->chains.size(); k++) {
         (void)hipEventRecord(b->chains[k]->joined, b->chains[k]->stream);
@@ -384,7 +385,7 @@ int captureGraphs(hvvr_gpu_batch* b, hvvr_gpu_scene* s) {
     for (size_t k = 0; k < b->chains.size(); k++) {
         Chain& c = *b->chains[k];
         hipStream_t st = c.stream ? c.stream : b->stream;
-        int rc = capture(st, [&] { enqueueChain(b, c, s->textureCount > 0); }, b->graphs[k], b->execs[k]);
+        int rc = capture(st, [&] { enqueueChain(b, c, s); }, b->graphs[k], b->execs[k]);
         if (rc)
             return rc;
     }

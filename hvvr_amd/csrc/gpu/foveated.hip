@@ -315,7 +315,7 @@ struct BlurArgs {
 // FinishConstrastEnhancement of the pixel against its filtered value as stored, which needs
 // no neighbour. A pixel's time is its powers: the eleven taps' weights are five (a tap and
 // its opposite share one, the centre's is 1), the encoding takes three. Both passes and the
-// contrast of a 1080x1200 image take 0.125 ms, 0.197 with a power and a division per tap and
+// contrast of a 1080x1200 image take 0.128 ms, 0.197 with a power and a division per tap and
 // the contrast in a launch of its own.
 template <bool Contrast>
 __global__ __launch_bounds__(256) void eccentricityBlurKernel(BlurArgs a) {

@@ -1,11 +1,12 @@
 // Triangle-list intersection for one view (raycaster/intersect.cu:117-342 with the
-// primitive tests of raycaster/prim_tests.h:18-231), one 128-thread workgroup per tile
-// (= two wave64s), one thread per sample, A subsamples per thread.
+// primitive tests of raycaster/prim_tests.h:18-231), one workgroup of W waves per tile. The
+// tile's 128 samples are two waves' lanes; each sample's A subsamples are split in S shares
+// of P, one for each of S pairs of waves; waves beyond 2 * S only cull.
 //
-// Per tile the list is processed in chunks of 128 entries. Each thread culls one
+// Per tile the list is processed in chunks of 64 * W entries. Each thread culls one
 // triangle against the tile (4 frustum planes, back-face/behind-origin, 4-corner
 // barycentric range); survivors are compacted into LDS in list order with a 64-bit
-// wave ballot + popcount and a two-wave prefix; then every thread tests its A
+// wave ballot + popcount and a prefix over the waves; then every thread tests its P
 // subsamples against every survivor in order, keeping the nearest hit. The per-tile
 // triangle setup (edges, normal, origin offset, plane distance t) is computed once
 // by the culling thread and shared through LDS, so the per-sample loop reads it with
@@ -322,25 +323,40 @@ __device__ inline bool missedByAll(const Tri& c, const WaveBundle& w) {
     return v0 || w0 || u0;
 }
 
-template <int A, bool DoF>
+template <int A, bool DoF, int S, int W>
 __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
     using Cached = typename std::conditional<DoF, TriTileDoF, TriTile>::type;
-    __shared__ Cached cache[128];
+    static_assert(A % S == 0 && W >= 2 * S, "a wave for every share of the subsamples");
+    constexpr uint32_t Threads = 64u * W;
+    constexpr int P = A / S; // subsamples per lane
+    // the survivors; after the last of them every subsample's hit, where several waves share
+    // a sample's
+    constexpr size_t HitBytes = S > 1 ? sizeof(uint32_t) * A * TILE_SIZE : 0;
+    __shared__ __attribute__((aligned(16))) char shared[sizeof(Cached) * Threads > HitBytes ? sizeof(Cached) * Threads : HitBytes];
+    Cached* const cache = reinterpret_cast<Cached*>(shared);
     __shared__ DofTile dofTile;
-    __shared__ uint32_t cacheIndex[128];
+    __shared__ uint32_t cacheIndex[Threads];
     __shared__ float planes[4][4];
     __shared__ SimpleRayFrustum frustum;
-    __shared__ uint32_t waveSurvivors[2];
+    __shared__ uint32_t waveSurvivors[W];
 
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
+    const uint32_t lane = tid & 63u, wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
     uint32_t listCount = args.tileCounts[tile];
     const uint32_t listStart = args.tileOffsets[tile];
     // a list that did not fit the list budget is skipped (the traversal raised the
     // overflow flag, and the frame reports an error)
     if (uint64_t(listStart) + listCount > args.listCapacity)
         listCount = 0;
-    const uint32_t sample = tile * TILE_SIZE + tid;
+    // a wave beyond the samples' two with nothing of the list to cull ends here (a barrier
+    // waits for the waves still running)
+    const bool tests = W == 2 * S || wave < 2u * S;
+    if (!tests && wave * 64u >= listCount)
+        return;
+    const uint32_t waves = listCount >= Threads ? uint32_t(W) : listCount <= 128u * S ? 2u * S : (listCount + 63u) / 64u;
+    const int first = int(wave >> 1) * P; // this wave's first subsample
+    const uint32_t inTile = tid & (TILE_SIZE - 1u);
+    const uint32_t sample = tile * TILE_SIZE + inTile;
 
     const matrix4x4& m = args.cameraToWorld;
     const matrix3x3 rot = m.upper3x3();
@@ -358,7 +374,7 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
         if (tid == 64)
             dofTile = dofTileLoad(rot, beam, args.lensRadius, args.focalDistance);
         lcfc = dofLensToFocal(rot, rot * beam.centerRay, args.focalDistance);
-        lensBase = (args.occRank[tile] % DOF_LENS_TABLE_ROWS) * TILE_SIZE * A + tid;
+        lensBase = (args.occRank[tile] % DOF_LENS_TABLE_ROWS) * TILE_SIZE * A + inTile;
     }
 
     if (tid == 0) {
@@ -375,21 +391,23 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
 
     // depth of field: the lens position of each subsample (up to eight in registers), read
     // from the tile's lens-table row
-    constexpr int LensRegs = DoF && A <= 8 ? A : 1;
+    constexpr int LensRegs = DoF && P <= 8 ? P : 1;
     vector2 lensReg[LensRegs];
     auto lensUV = [&](int i) {
-        if constexpr (DoF && A <= 8)
+        if constexpr (DoF && P <= 8)
             return lensReg[i];
         else
-            return args.lensTable[lensBase + i * TILE_SIZE];
+            return args.lensTable[lensBase + (first + i) * TILE_SIZE];
     };
-    if constexpr (DoF && A <= 8) {
+    if constexpr (DoF && P <= 8) {
+        if (tests) {
 #pragma unroll
-        for (int i = 0; i < A; i++)
-            lensReg[i] = args.lensTable[lensBase + i * TILE_SIZE];
+            for (int i = 0; i < P; i++)
+                lensReg[i] = args.lensTable[lensBase + (first + i) * TILE_SIZE];
+        }
     }
     // each wave's ray bundle for the occlusion skip, kept in LDS (read once per 64 survivors)
-    __shared__ WaveBundle bundles[2];
+    __shared__ WaveBundle bundles[2 * S];
     // this lane's centre ray and the reach of its subsamples from it
     auto laneRays = [&](vector3& d, vector3& s) {
         float du = args.offsetMax.x, dv = args.offsetMax.y;
@@ -400,8 +418,8 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
             u = dofTile.lensU;
             v = dofTile.lensV;
             du = dv = 0.0f;
-            for (int i = 0; i < A; i++) {
-                const vector2 dirUV = dofDirUV(args.offsets[i], dofTile.focalToLensScale, lensUV(i));
+            for (int i = 0; i < P; i++) {
+                const vector2 dirUV = dofDirUV(args.offsets[first + i], dofTile.focalToLensScale, lensUV(i));
                 du = fmaxf(du, fabsf(dirUV.x));
                 dv = fmaxf(dv, fabsf(dirUV.y));
             }
@@ -422,16 +440,16 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
     };
     if constexpr (DoF)
         __syncthreads(); // the tile's lens frame is there
-    {
+    if (tests) {
         const WaveBundle b = bundleOf(true);
         if (lane == 0)
             bundles[wave] = b;
     }
 
-    float depth[A];
-    uint32_t hit[A];
+    float depth[P];
+    uint32_t hit[P];
 #pragma unroll
-    for (int i = 0; i < A; i++) {
+    for (int i = 0; i < P; i++) {
         depth[i] = FLT_MAX;
         hit[i] = badTriIndex;
     }
@@ -440,7 +458,7 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
     uint32_t survivorsSum = 0;
     // survivors this wave tested (wave-uniform: a scalar register)
     uint32_t testedSum = 0;
-    for (uint32_t chunk = 0; chunk < listCount; chunk += 128) {
+    for (uint32_t chunk = 0; chunk < listCount; chunk += Threads) {
         // ---- cull one list entry per thread ----
         bool keep = false;
         uint32_t triIndex = badTriIndex;
@@ -482,9 +500,15 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
         if (lane == 0)
             waveSurvivors[wave] = uint32_t(__popcll(ballot));
         __syncthreads();
-        uint32_t total = waveSurvivors[0] + waveSurvivors[1];
+        uint32_t total = 0, before = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < uint32_t(W); k++) {
+            const uint32_t c = k < waves ? waveSurvivors[k] : 0u;
+            before += k < wave ? c : 0u;
+            total += c;
+        }
         if (keep) {
-            uint32_t slot = (wave ? waveSurvivors[0] : 0u) + prefix;
+            uint32_t slot = before + prefix;
             cache[slot] = tt;
             cacheIndex[slot] = triIndex;
         }
@@ -496,11 +520,11 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
         auto farthest = [&] {
             float far = depth[0];
 #pragma unroll
-            for (int i = 1; i < A; i++)
+            for (int i = 1; i < P; i++)
                 far = fmaxf(far, depth[i]);
             return far;
         };
-        for (uint32_t j0 = 0; j0 < total; j0 += 64) {
+        for (uint32_t j0 = 0; tests && j0 < total; j0 += 64) {
             // lane k's survivor, and which of the 64 the wave's rays may reach
             const uint32_t n = total - j0 < 64u ? total - j0 : 64u;
             uint64_t todo = n == 64u ? ~0ull : (1ull << n) - 1ull;
@@ -527,9 +551,9 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
                         // IntersectTriangleThreadDoF (prim_tests.h:295-355)
                         const float denomCenter = dot(-lcfc, c.normal);
 #pragma unroll
-                        for (int i = 0; i < A; i++) {
+                        for (int i = 0; i < P; i++) {
                             const vector2 uv = lensUV(i);
-                            const vector2 dirUV = dofDirUV(args.offsets[i], dofTile.focalToLensScale, uv);
+                            const vector2 dirUV = dofDirUV(args.offsets[first + i], dofTile.focalToLensScale, uv);
                             if (dofTest(c, denomCenter, lcfc, dofTile.lensU, dofTile.lensV, uv, dirUV, depth[i]))
                                 hit[i] = idx;
                         }
@@ -547,9 +571,9 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
                         const float dW0 = -dot(c.e0, cu), dW1 = -dot(c.e0, cv);
                         const float t = c.t;
 #pragma unroll
-                        for (int i = 0; i < A; i++) {
+                        for (int i = 0; i < P; i++) {
                             // IntersectTriangleThread::test (prim_tests.h:192-231)
-                            const vector2 a = args.offsets[i];
+                            const vector2 a = args.offsets[first + i];
                             const float denom = fmaf(dD1, a.y, fmaf(dD0, a.x, denomCenter));
                             const float depthDelta = fmaf(depth[i], denom, -t);
                             const float v = fmaf(dV1, a.y, fmaf(dV0, a.x, vCenter));
@@ -569,12 +593,18 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
         }
         __syncthreads(); // before the next chunk overwrites the cache
     }
+    if (!tests)
+        return;
     if (lane == 0)
         waveSurvivors[wave] = testedSum; // the loop's last read of it preceded a barrier
     __syncthreads();
     if (tid == 0) {
         args.tileSurvivors[tile] = survivorsSum;
-        args.tileTested[tile] = waveSurvivors[0] + waveSurvivors[1];
+        uint32_t tested = 0;
+#pragma unroll
+        for (int k = 0; k < 2 * S; k++)
+            tested += waveSurvivors[k];
+        args.tileTested[tile] = (tested + S - 1) / S; // each of them for a part of the subsamples
     }
 
     if (args.hits) {
@@ -582,22 +612,22 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
         // and its barycentrics on that subsample's ray (calcUVW, prim_tests.h:233-245, or
         // its thin-lens twin :366-392), recomputed here from the winning triangle. The
         // first pass parks (depth, id) in the output so the second need not be unrolled.
-        vector4* out = args.hits + size_t(sample) * A;
+        vector4* out = args.hits + size_t(sample) * A + first;
 #pragma unroll
-        for (int i = 0; i < A; i++)
+        for (int i = 0; i < P; i++)
             out[i] = vector4(depth[i], __uint_as_float(hit[i]), 0.0f, 0.0f);
-        for (int i = 0; i < A; i++) {
+        for (int i = 0; i < P; i++) {
             const vector4 h = out[i];
             const uint32_t id = __float_as_uint(h.y);
             float bx = 0.0f, by = 0.0f, bz = 0.0f;
             if (id != badTriIndex) {
                 const PrecomputedTriangleIntersect T = args.tris[id];
                 if constexpr (DoF) {
-                    const vector2 lensUV = args.lensTable[lensBase + i * TILE_SIZE];
-                    const vector2 dirUV = dofDirUV(args.offsets[i], dofTile.focalToLensScale, lensUV);
+                    const vector2 lensUV = args.lensTable[lensBase + (first + i) * TILE_SIZE];
+                    const vector2 dirUV = dofDirUV(args.offsets[first + i], dofTile.focalToLensScale, lensUV);
                     dofUVW(T, rayOrigin, dofTile, lcfc, lensUV.x, lensUV.y, dirUV.x, dirUV.y, bx, by, bz);
                 } else {
-                    pinholeUVW(T, rayOrigin, ndir, ndu, ndv, args.offsets[i].x, args.offsets[i].y, bx, by, bz);
+                    pinholeUVW(T, rayOrigin, ndir, ndu, ndv, args.offsets[first + i].x, args.offsets[first + i].y, bx, by, bz);
                 }
             }
             out[i] = vector4(h.x, bx, by, bz);
@@ -605,7 +635,23 @@ __device__ inline void intersectBody(const IntersectArgs& args, uint32_t tile) {
     }
 
     GBufferSubsample* waveBase = args.gbuffer + size_t(sample >> 6) * 64 * A;
-    emitGBuffer<A>(hit, waveBase, lane);
+    if constexpr (S == 1) {
+        emitGBuffer<A>(hit, waveBase, lane);
+    } else {
+        // the first two waves collect the tile's hits (where the survivors were)
+        uint32_t* all = reinterpret_cast<uint32_t*>(shared);
+#pragma unroll
+        for (int i = 0; i < P; i++)
+            all[uint32_t(first + i) * TILE_SIZE + inTile] = hit[i];
+        __syncthreads();
+        if (wave >= 2u)
+            return;
+        uint32_t every[A];
+#pragma unroll
+        for (int i = 0; i < A; i++)
+            every[i] = all[uint32_t(i) * TILE_SIZE + inTile];
+        emitGBuffer<A>(every, waveBase, lane);
+    }
 }
 
 // Waves per SIMD the register allocator is held to: as many as it reaches without spills of
@@ -617,21 +663,47 @@ constexpr int intersectWaves(int A, bool DoF) {
     return DoF ? (A <= 4 ? 4 : A == 8 ? 3 : 1) : (A <= 4 ? 5 : A == 8 ? 4 : 1);
 }
 
-template <int A, bool DoF>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(intersectWaves(A, DoF))))
+// How a tile's workgroup is split: Split shares of every sample's subsamples, Waves waves.
+//  Narrow: the tile's two waves of samples do everything.
+//  Deep: two more cull only. For long lists, which one workgroup walks Waves * 64 entries at
+//    a time: a 2M-triangle 760x840 view, its mean list 2640 entries, 0.206 -> 0.197 ms, a
+//    batch of 16 views of 1M triangles, 2000 to 10000 entries a tile, 6.76 -> 6.30 ms.
+//    Shorter lists lose by the waves that wait while two test: a 1M-triangle 1080x1200 view,
+//    1095 entries, 0.195 -> 0.208 ms, so the line is 256 scene triangles a tile (the first
+//    has 420, the last 103).
+//  Wide: up to eight waves, four shares. Where the tiles do not fill the chip the slowest
+//    one sets the time (a few hundred survivors tested one after another at up to 1400
+//    cycles each, lists of up to 15000 entries against a mean of 2500): 257x303 8x, 640
+//    tiles, 0.253 -> 0.159 ms; 540x600 8x thin lens, 2560 tiles, 0.207 -> 0.137; foveated
+//    eyes of 2496 tiles, 4x thin lens 0.469 -> 0.301 and 2x of 1M triangles 0.444 -> 0.305.
+//    A view of 4992 tiles gains nothing and one of 10176 takes 0.228 ms instead of 0.107:
+//    the line is the tiles whose two waves are on the chip at once, five a SIMD. With short
+//    lists the waves are not worth their start (640x480 1x, 36 entries a tile, 3 scene
+//    triangles: 0.0194 -> 0.0226 ms): Wide from 32 scene triangles a tile.
+constexpr uint64_t kDeepTriangles = 256;
+enum class TileShape { Narrow, Deep, Wide };
+constexpr int intersectSplit(int A, TileShape shape) { return shape != TileShape::Wide ? 1 : A < 4 ? A : 4; }
+constexpr int intersectBlockWaves(int A, TileShape shape) {
+    return shape == TileShape::Narrow ? 2 : shape == TileShape::Wide && A >= 4 ? 8 : 4;
+}
+
+template <int A, bool DoF, TileShape Shape>
+__global__ __launch_bounds__(64 * intersectBlockWaves(A, Shape))
+__attribute__((amdgpu_waves_per_eu(intersectWaves(A / intersectSplit(A, Shape), DoF))))
 void intersectKernel(IntersectArgs args) {
-    intersectBody<A, DoF>(args, blockIdx.x);
+    intersectBody<A, DoF, intersectSplit(A, Shape), intersectBlockWaves(A, Shape)>(args, blockIdx.x);
 }
 
 // every tile of the views whose units `start` lists (pinhole views of one MSAA rate)
-template <int A>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(intersectWaves(A, false))))
-void intersectBatchKernel(const IntersectArgs* __restrict__ all,
-                                                            const uint32_t* __restrict__ start, uint32_t n,
-                                                            uint32_t swizzle) {
+template <int A, TileShape Shape>
+__global__ __launch_bounds__(64 * intersectBlockWaves(A, Shape))
+__attribute__((amdgpu_waves_per_eu(intersectWaves(A / intersectSplit(A, Shape), false))))
+void intersectBatchKernel(const IntersectArgs* __restrict__ all, const uint32_t* __restrict__ start, uint32_t n,
+                          uint32_t swizzle) {
     const uint32_t unit = xcdUnit(blockIdx.x, gridDim.x, swizzle);
     const uint32_t v = batchView(start, n, unit);
-    intersectBody<A, false>(batchArgs(all, v), unit - start[v]);
+    intersectBody<A, false, intersectSplit(A, Shape), intersectBlockWaves(A, Shape)>(batchArgs(all, v),
+                                                                                     unit - start[v]);
 }
 
 IntersectArgs intersectArgs(const hvvr_gpu_view* v, const hvvr_gpu_scene* s, const matrix4x4& m) {
@@ -665,15 +737,28 @@ IntersectArgs intersectArgs(const hvvr_gpu_view* v, const hvvr_gpu_scene* s, con
 
 void launchIntersect(hvvr_gpu_view* v, const hvvr_gpu_scene* s, const matrix4x4& m, hipStream_t stream) {
     const IntersectArgs a = intersectArgs(v, s, m);
-    dim3 grid(v->tileCount), block(128);
-    const bool dof = v->dof;
+    const dim3 grid(v->tileCount);
+    const uint64_t triangles = s->triangleCount, tiles = v->tileCount;
+    const TileShape shape = tiles <= 2560u && triangles >= 32u * tiles        ? TileShape::Wide
+                            : !v->dof && triangles >= kDeepTriangles * tiles ? TileShape::Deep
+                                                                              : TileShape::Narrow;
     switch (v->msaaRate) {
+#define HVVR_INTERSECT_SHAPE(A, DoF, Shape) \
+    intersectKernel<A, DoF, TileShape::Shape><<<grid, 64 * intersectBlockWaves(A, TileShape::Shape), 0, stream>>>(a)
 #define HVVR_INTERSECT_CASE(A)                                                        \
     case A:                                                                           \
-        if (dof)                                                                      \
-            intersectKernel<A, true><<<grid, block, 0, stream>>>(a);                  \
-        else                                                                          \
-            intersectKernel<A, false><<<grid, block, 0, stream>>>(a);                 \
+        if (shape == TileShape::Wide) {                                               \
+            if (v->dof)                                                               \
+                HVVR_INTERSECT_SHAPE(A, true, Wide);                                  \
+            else                                                                      \
+                HVVR_INTERSECT_SHAPE(A, false, Wide);                                 \
+        } else if (v->dof) {                                                          \
+            HVVR_INTERSECT_SHAPE(A, true, Narrow);                                    \
+        } else if (shape == TileShape::Deep) {                                        \
+            HVVR_INTERSECT_SHAPE(A, false, Deep);                                     \
+        } else {                                                                      \
+            HVVR_INTERSECT_SHAPE(A, false, Narrow);                                   \
+        }                                                                             \
         break;
         HVVR_INTERSECT_CASE(1)
         HVVR_INTERSECT_CASE(2)
@@ -682,16 +767,25 @@ void launchIntersect(hvvr_gpu_view* v, const hvvr_gpu_scene* s, const matrix4x4&
         HVVR_INTERSECT_CASE(16)
         HVVR_INTERSECT_CASE(32)
 #undef HVVR_INTERSECT_CASE
+#undef HVVR_INTERSECT_SHAPE
         default: break;
     }
 }
 
 void launchIntersectBatch(int msaaRate, const IntersectArgs* all, const uint32_t* start, uint32_t viewCount,
-                          uint32_t units, const LaunchShape& shape, hipStream_t stream) {
+                          uint32_t units, uint32_t triangles, const LaunchShape& shape, hipStream_t stream) {
+    const bool deep = uint64_t(triangles) * viewCount >= kDeepTriangles * units;
     switch (msaaRate) {
+#define HVVR_INTERSECT_BATCH_SHAPE(A, Shape)                                                                  \
+    intersectBatchKernel<A, TileShape::Shape>                                                                 \
+        <<<units, 64 * intersectBlockWaves(A, TileShape::Shape), 0, stream>>>(all, start, viewCount,          \
+                                                                              shape.xcdSwizzle)
 #define HVVR_INTERSECT_BATCH_CASE(A)                                                                          \
     case A:                                                                                                   \
-        intersectBatchKernel<A><<<units, 128, 0, stream>>>(all, start, viewCount, shape.xcdSwizzle);          \
+        if (deep)                                                                                             \
+            HVVR_INTERSECT_BATCH_SHAPE(A, Deep);                                                              \
+        else                                                                                                  \
+            HVVR_INTERSECT_BATCH_SHAPE(A, Narrow);                                                            \
         break;
         HVVR_INTERSECT_BATCH_CASE(1)
         HVVR_INTERSECT_BATCH_CASE(2)
@@ -700,6 +794,7 @@ void launchIntersectBatch(int msaaRate, const IntersectArgs* all, const uint32_t
         HVVR_INTERSECT_BATCH_CASE(16)
         HVVR_INTERSECT_BATCH_CASE(32)
 #undef HVVR_INTERSECT_BATCH_CASE
+#undef HVVR_INTERSECT_BATCH_SHAPE
         default: break;
     }
 }

@@ -179,8 +179,9 @@ void launchTileListsBatch(const TileListArgs* all, const uint32_t* start, uint32
                           const LaunchShape& shape, hipStream_t stream);
 void launchTileWalkBatch(const TileWalkArgs* all, uint32_t viewCount, uint32_t maxTiles, const LaunchShape& shape,
                          hipStream_t stream);
+// triangles: the scene's (with the units, how long the tiles' lists get)
 void launchIntersectBatch(int msaaRate, const IntersectArgs* all, const uint32_t* start, uint32_t viewCount,
-                          uint32_t units, const LaunchShape& shape, hipStream_t stream);
+                          uint32_t units, uint32_t triangles, const LaunchShape& shape, hipStream_t stream);
 // tex: the scene has textures (the resolve variant that reads them)
 void launchResolveBatch(int msaaRate, bool half, bool tex, const ResolveArgs* all, const uint32_t* start,
                         uint32_t viewCount, uint32_t units, const LaunchShape& shape, hipStream_t stream);

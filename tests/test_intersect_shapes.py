@@ -1,0 +1,89 @@
+"""The intersect's workgroup shapes (hvvr_amd/csrc/gpu/intersect.hip) at the edges of a tile's
+list: 64 entries a wave, 256 and 512 a workgroup, lists that leave whole waves without an
+entry, several rounds, and every split of the subsamples, pinhole and thin lens, against the
+oracle: ids, masks, depths and barycentrics bit-exact. The scene holds `n` triangles as wide
+as the view, so that a tile's list has nearly all of them, and others behind the camera up to
+`total`, which picks the shape (the view has 64 tiles)."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LENS = (0.05, 8.0)
+
+
+def _soup(H, n, total):
+    rng = np.random.default_rng(n)
+    v = np.zeros(3 * total, H.DTYPES["vertex"])
+    centre = rng.uniform([-2, -2, -20], [2, 2, -4], (total, 1, 3))
+    centre[n:, 0, 2] += 60
+    v["pos"] = (centre + rng.uniform(-3, 3, (total, 3, 3)) * [1, 1, 0.2]).reshape(-1, 3)
+    v["normal"][:, 2] = np.float16(1).view(np.uint16)
+    m = np.zeros(1, H.DTYPES["material"])
+    m["diffuse"] = (0.5, 0.5, 0.5, 1)
+    m["textureIDsAndShadingModel"] = 1 | (0xFFFF << 16) | (0xFFFF << 32) | (0xFFFF << 48)
+    tri = np.arange(3 * total, dtype=np.uint32).reshape(total, 3)
+    return H.HostScene.from_meshes([(v, tri, np.zeros(total, np.uint32), None)], m)
+
+
+def _view(H, lens=False):
+    w, h, t = 32, 24, 0.35
+    s = H.grid_samples(w, h)
+    if lens:
+        return H.HostView.from_samples(s, w, h, (-t, -t, t, t), lens_radius=LENS[0], focal_distance=LENS[1])
+    return H.HostView.from_samples(s, w, h, (-t, -t, t, t))
+
+
+def _check(H, O, gv, ref, view, A, m, dof):
+    counts, lists = gv.read_tile_lists()
+    assert np.array_equal(counts, ref["counts"]) and np.array_equal(lists, ref["lists"])
+    tri, mask = gv.read_gbuffer()
+    rtri, rmask = O.gbuffer_slots(ref["tri_ids"])
+    assert np.array_equal(tri, rtri) and np.array_equal(mask, rmask)
+    got = gv.read_hits()
+    want = O.hits_view(view.beams, m, ref["offsets"], A, ref["tri_ids"], ref["tris"], ref["counts"], dof)
+    assert np.array_equal(got[..., 0].view(np.uint32), ref["depth"].reshape(-1, A).view(np.uint32))
+    assert np.array_equal(got[..., 1:].view(np.uint32), want.view(np.uint32))
+    st = gv.stats()
+    assert st.survivorPairs == ref["survivors"] and st.testedPairs <= st.survivorPairs
+
+
+# two waves a tile below 32 triangles a tile, up to eight from there on
+@pytest.mark.parametrize("n,total", [(300, 2047), (1, 2048), (63, 2048), (65, 2048), (257, 2048), (511, 2048),
+                                     (514, 2048), (1300, 2048)])
+@pytest.mark.parametrize("A,lens", [(1, False), (2, False), (4, False), (8, False), (16, False), (32, False),
+                                    (1, True), (2, True), (8, True), (32, True)])
+def test_single_view(H, O, ctx, n, total, A, lens):
+    scene, view = _soup(H, n, total), _view(H, lens)
+    assert view.tile_count == 64
+    m = np.eye(4, dtype=np.float32).reshape(16)
+    ref = O.render_view(scene, view, A, camera_to_world=m, with_colors=False)
+    assert ref["counts"].max() >= n // 2
+    gs, gv = H.GpuScene(ctx, scene), H.GpuView(ctx, view, A)
+    gv.set_hit_output(True)
+    gv.render(gs, m)
+    _check(H, O, gv, ref, view, A, m, (*LENS, H.lens_table(A)) if lens else None)
+    gv.close()
+    gs.close()
+
+
+# one view of each rate: two waves a tile below 256 triangles a tile, four from there on
+@pytest.mark.parametrize("n,total", [(300, 16383), (1, 16384), (129, 16384), (257, 16384), (700, 16384)])
+def test_batch(H, O, ctx, n, total):
+    scene, view = _soup(H, n, total), _view(H)
+    m = np.eye(4, dtype=np.float32).reshape(16)
+    rates = [1, 2, 4, 8]
+    gs = H.GpuScene(ctx, scene)
+    views = [H.GpuView(ctx, view, A) for A in rates]
+    for v in views:
+        v.set_hit_output(True)
+    batch = H.GpuBatch(ctx, views)
+    batch.render(gs, np.stack([m] * len(rates)))
+    batch.synchronize()
+    for v, A in zip(views, rates):
+        _check(H, O, v, O.render_view(scene, view, A, camera_to_world=m, with_colors=False), view, A, m, None)
+    batch.close()
+    for v in views:
+        v.close()
+    gs.close()
