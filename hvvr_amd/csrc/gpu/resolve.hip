@@ -1,8 +1,8 @@
 // Resolve (MSAA GGX shading, ACES tone map, sRGB8) and remap for one view.
 //
 //   resolveKernel  ResolveKernel + ShadeMSAA (raycaster/resolve.cu:161-284, 324-384) and
-//                  ClearEmptyKernel (resolve.cu:527-542) in one launch: one 128-thread
-//                  workgroup per tile, one thread per sample; tiles whose triangle list
+//                  ClearEmptyKernel (resolve.cu:527-542) in one launch: one workgroup per
+//                  tile, its lanes over the samples' triangles; tiles whose triangle list
 //                  was empty write the clear colour 0xff000000 without touching the
 //                  GBuffer. Per unique triangle of a sample: centroid of its subsample
 //                  offsets, barycentrics (calcUVW, prim_tests.h:233-245), vertex
@@ -278,114 +278,221 @@ __device__ inline float acesFilm(float x) {
     return saturate((x * (a * x + b)) * rcpFast(x * (c * x + d) + e));
 }
 
+// A sample's rays, and its thin lens
+struct ResolveRays {
+    vector3 ndir, ndu, ndv;
+    vector3 lcfc;      // depth of field: the per-sample focal offset
+    uint32_t lensBase; // and its place in the tile's lens-table row
+};
+
+template <int A, bool DoF>
+__device__ inline ResolveRays resolveRays(const ResolveArgs& args, const matrix3x3& rot,
+                                          const DirectionalBeam& beam, uint32_t tile, uint32_t inTile) {
+    ResolveRays r;
+    r.ndir = -(rot * beam.centerRay);
+    r.ndu = -(rot * beam.du);
+    r.ndv = -(rot * beam.dv);
+    r.lcfc = vector3(0.0f);
+    r.lensBase = 0;
+    if constexpr (DoF) {
+        r.lcfc = dofLensToFocal(rot, rot * beam.centerRay, args.focalDistance);
+        r.lensBase = (args.occRank[tile] % DOF_LENS_TABLE_ROWS) * TILE_SIZE * A + inTile;
+    }
+    return r;
+}
+
+// The colour of one triangle of a sample.
 // Tex: the scene has textures (a variant of its own: the texture reads' registers would
 // cost untextured scenes occupancy)
+template <bool DoF, bool Half, bool Tex>
+__device__ inline vector3 shadeSlot(const ResolveArgs& args, const vector3& cam, const DofTile& dofTile,
+                                    const ResolveRays& r, const GBufferSubsample& g) {
+    const uint32_t mask = g.sampleMask;
+    float inv = 1.0f / float(__popc(mask));
+    float cx = 0.0f, cy = 0.0f;
+    float lx = 0.0f, ly = 0.0f, dx = 0.0f, dy = 0.0f;
+    for (uint32_t bits = mask; bits; bits &= bits - 1) {
+        int i = __ffs(bits) - 1;
+        vector2 o = args.offsets[i];
+        cx = cx + o.x * inv;
+        cy = cy + o.y * inv;
+        if constexpr (DoF) {
+            // centroid lens position and direction offset (resolve.cu:212-222)
+            const vector2 lensUV = args.lensTable[r.lensBase + i * TILE_SIZE];
+            const vector2 dirUV = dofDirUV(o, dofTile.focalToLensScale, lensUV);
+            lx = lx + lensUV.x * inv;
+            ly = ly + lensUV.y * inv;
+            dx = dx + dirUV.x * inv;
+            dy = dy + dirUV.y * inv;
+        }
+    }
+    PrecomputedTriangleIntersect T = args.tris[g.triIndex];
+    float bx, by, bz;
+    if constexpr (DoF)
+        dofUVW(T, cam, dofTile, r.lcfc, lx, ly, dx, dy, bx, by, bz); // at the centroid
+    else
+        pinholeUVW(T, cam, r.ndir, r.ndu, r.ndv, cx, cy, bx, by, bz);
+    PrecomputedTriangleShade S = args.triShade[g.triIndex];
+    ShadingVertex V0 = args.verts[S.indices[0]], V1 = args.verts[S.indices[1]], V2 = args.verts[S.indices[2]];
+    vector3 pos = V0.pos * bx + V1.pos * by + V2.pos * bz;
+    vector3 n0(halfToFloat(V0.normal[0]), halfToFloat(V0.normal[1]), halfToFloat(V0.normal[2]));
+    vector3 n1(halfToFloat(V1.normal[0]), halfToFloat(V1.normal[1]), halfToFloat(V1.normal[2]));
+    vector3 n2(halfToFloat(V2.normal[0]), halfToFloat(V2.normal[1]), halfToFloat(V2.normal[2]));
+    vector3 nrm = n0 * bx + n1 * by + n2 * bz;
+    const SimpleMaterial& mat = args.materials[S.material];
+    const bool textured = Tex && materialTextured(mat, args.tex);
+    vector2 uv(0.0f), dUVdX(0.0f), dUVdY(0.0f);
+    if (textured) {
+        // UV derivatives (resolve.cu:258-275): barycentrics one unit along each
+        // subsample axis from the centroid (for depth of field, along each axis of the
+        // focal-plane offset)
+        float xb0, xb1, xb2, yb0, yb1, yb2;
+        if constexpr (DoF) {
+            dofUVW(T, cam, dofTile, r.lcfc, lx, ly, dx + 1.0f, dy, xb0, xb1, xb2);
+            dofUVW(T, cam, dofTile, r.lcfc, lx, ly, dx, dy + 1.0f, yb0, yb1, yb2);
+        } else {
+            pinholeUVW(T, cam, r.ndir, r.ndu, r.ndv, cx + 1.0f, cy, xb0, xb1, xb2);
+            pinholeUVW(T, cam, r.ndir, r.ndu, r.ndv, cx, cy + 1.0f, yb0, yb1, yb2);
+        }
+        uv = V0.uv * bx + V1.uv * by + V2.uv * bz;
+        dUVdX = (V0.uv * xb0 + V1.uv * xb1 + V2.uv * xb2) - uv;
+        dUVdY = (V0.uv * yb0 + V1.uv * yb1 + V2.uv * yb2) - uv;
+    }
+    vector3 c;
+    if (textured) {
+        const SurfaceInputs in = surfaceInputs(mat, args.tex, uv, dUVdX, dUVdY);
+        c = Half ? ggxShadeHalf(in, pos, nrm, cam, args.env) : ggxShade(in, pos, nrm, cam, args.env);
+    } else {
+        const MaterialInputs in{mat};
+        c = Half ? ggxShadeHalf(in, pos, nrm, cam, args.env) : ggxShade(in, pos, nrm, cam, args.env);
+    }
+    return c;
+}
+
+// The triangles of a tile's samples are shaded by whichever lane is next, not by their
+// sample's: a sample on an edge has several, most one, and in a loop over a sample's own the
+// wave took as many turns as its busiest lane and a small view's few waves one turn after
+// another. The (slot, sample) pairs are gathered in LDS, slot by slot, the lanes shade them
+// in turn, and each sample adds its colours up in slot order. Bound by the shading's
+// arithmetic and the vertex and texel gathers: a textured 257x303 8x view 0.241 -> 0.078 ms
+// (two waves 0.131, eight 0.046, but eight lose at 1080x1200 8x textured: 0.274 -> 0.187 with
+// two or four, 0.243 with eight), 1080x1200 4x textured 0.230 -> 0.185, 540x600 8x thin lens
+// 0.048 -> 0.031 (eight 0.038), 1080x1200 4x room eye 0.065 -> 0.057 (four waves 0.061).
+// 16x and 32x, whose colours would take 28 and 57 KB of LDS, loop over a sample's own
+// triangles, and so does 1x, which has one.
+constexpr bool resolveGathers(int A) { return A >= 2 && A <= 8; }
+constexpr int resolveWaves(int A) { return A == 8 ? 4 : 2; }
+
 template <int A, bool DoF, bool Half, bool Tex>
 __device__ inline void resolveBody(const ResolveArgs& args, uint32_t tile) {
+    constexpr bool Gather = resolveGathers(A);
+    constexpr uint32_t Threads = 64u * resolveWaves(A);
     __shared__ DofTile dofTile;
+    __shared__ float colours[Gather ? 3 * A * TILE_SIZE : 1];
+    __shared__ uint16_t items[Gather ? A * TILE_SIZE : 1]; // slot * 128 + sample of the tile
+    __shared__ uint32_t itemCount;
     const uint32_t tid = threadIdx.x;
-    const uint32_t sample = tile * TILE_SIZE + tid;
+    const bool owner = Threads == TILE_SIZE || tid < TILE_SIZE;
+    const uint32_t inTile = tid & (TILE_SIZE - 1u);
+    const uint32_t sample = tile * TILE_SIZE + inTile;
     if (args.tileCounts[tile] == 0) {
         // ClearEmptyKernel (resolve.cu:527-542)
-        args.sampleResults[sample] = 0xff000000u;
-        if (args.tMax)
-            args.tMax[sample] = INFINITY;
+        if (owner) {
+            args.sampleResults[sample] = 0xff000000u;
+            if (args.tMax)
+                args.tMax[sample] = INFINITY;
+        }
         return;
     }
     const uint32_t lane = tid & 63u;
-    const GBufferSubsample* waveBase = args.gbuffer + size_t(sample >> 6) * 64 * A;
+    const GBufferSubsample* tileBase = args.gbuffer + size_t(tile) * TILE_SIZE * A;
+    const GBufferSubsample* waveBase = tileBase + (inTile >> 6) * 64 * A;
     const matrix4x4& m = args.cameraToWorld;
     const matrix3x3 rot = m.upper3x3();
     const vector3 cam = m.m3.xyz();
-    DirectionalBeam beam = args.beams[sample];
-    const vector3 ndir = -(rot * beam.centerRay);
-    const vector3 ndu = -(rot * beam.du);
-    const vector3 ndv = -(rot * beam.dv);
     const uint32_t maskAll = A < 32 ? ((1u << A) - 1u) : 0xffffffffu;
+    const DirectionalBeam beam = args.beams[sample];
     // depth of field: tile lens frame from sample 64 (ResolveKernel, resolve.cu:358-366),
     // per-sample focal offset, the lens-table row of this tile
-    vector3 lcfc(0.0f);
-    uint32_t lensBase = 0;
     if constexpr (DoF) {
         if (tid == 64)
             dofTile = dofTileLoad(rot, beam, args.lensRadius, args.focalDistance);
-        lcfc = dofLensToFocal(rot, rot * beam.centerRay, args.focalDistance);
-        lensBase = (args.occRank[tile] % DOF_LENS_TABLE_ROWS) * TILE_SIZE * A + tid;
-        __syncthreads();
     }
+    if (Gather && tid == 0)
+        itemCount = 0;
+    if constexpr (DoF || Gather)
+        __syncthreads();
 
     vector3 result(0.0f);
     uint32_t combined = 0;
     uint32_t tri0 = badTriIndex; // the triangle subsample 0 hit
-    for (int slot = 0; slot < A; slot++) {
+    // this sample's next triangle, false after the last
+    auto nextSlot = [&](int slot, GBufferSubsample& g) {
         if (combined == maskAll)
-            break;
-        GBufferSubsample g = waveBase[slot * 64 + lane];
+            return false;
+        g = waveBase[slot * 64 + lane];
         if (g.triIndex == badTriIndex)
-            break;
-        uint32_t mask = g.sampleMask;
-        combined |= mask;
-        if (mask & 1u)
+            return false;
+        combined |= g.sampleMask;
+        if (g.sampleMask & 1u)
             tri0 = g.triIndex;
-        float inv = 1.0f / float(__popc(mask));
-        float cx = 0.0f, cy = 0.0f;
-        float lx = 0.0f, ly = 0.0f, dx = 0.0f, dy = 0.0f;
-        for (uint32_t bits = mask; bits; bits &= bits - 1) {
-            int i = __ffs(bits) - 1;
-            vector2 o = args.offsets[i];
-            cx = cx + o.x * inv;
-            cy = cy + o.y * inv;
-            if constexpr (DoF) {
-                // centroid lens position and direction offset (resolve.cu:212-222)
-                const vector2 lensUV = args.lensTable[lensBase + i * TILE_SIZE];
-                const vector2 dirUV = dofDirUV(o, dofTile.focalToLensScale, lensUV);
-                lx = lx + lensUV.x * inv;
-                ly = ly + lensUV.y * inv;
-                dx = dx + dirUV.x * inv;
-                dy = dy + dirUV.y * inv;
+        return true;
+    };
+    if constexpr (Gather) {
+        uint8_t weight[A];
+        int slots = 0;
+        if (owner) {
+            bool more = true;
+#pragma unroll
+            for (int slot = 0; slot < A; slot++) {
+                GBufferSubsample g;
+                weight[slot] = 0;
+                more = more && nextSlot(slot, g);
+                const uint64_t with = __ballot(more);
+                if (with == 0ull)
+                    break;
+                uint32_t at = 0;
+                if (lane == 0)
+                    at = atomicAdd(&itemCount, uint32_t(__popcll(with)));
+                at = uint32_t(__builtin_amdgcn_readfirstlane(int(at)));
+                if (more) {
+                    items[at + __popcll(with & ((1ull << lane) - 1ull))] = uint16_t(slot * TILE_SIZE + inTile);
+                    weight[slot] = uint8_t(__popc(g.sampleMask));
+                    slots = slot + 1;
+                }
             }
         }
-        PrecomputedTriangleIntersect T = args.tris[g.triIndex];
-        float bx, by, bz;
-        if constexpr (DoF)
-            dofUVW(T, cam, dofTile, lcfc, lx, ly, dx, dy, bx, by, bz); // at the centroid
-        else
-            pinholeUVW(T, cam, ndir, ndu, ndv, cx, cy, bx, by, bz);
-        PrecomputedTriangleShade S = args.triShade[g.triIndex];
-        ShadingVertex V0 = args.verts[S.indices[0]], V1 = args.verts[S.indices[1]], V2 = args.verts[S.indices[2]];
-        vector3 pos = V0.pos * bx + V1.pos * by + V2.pos * bz;
-        vector3 n0(halfToFloat(V0.normal[0]), halfToFloat(V0.normal[1]), halfToFloat(V0.normal[2]));
-        vector3 n1(halfToFloat(V1.normal[0]), halfToFloat(V1.normal[1]), halfToFloat(V1.normal[2]));
-        vector3 n2(halfToFloat(V2.normal[0]), halfToFloat(V2.normal[1]), halfToFloat(V2.normal[2]));
-        vector3 nrm = n0 * bx + n1 * by + n2 * bz;
-        const SimpleMaterial& mat = args.materials[S.material];
-        const bool textured = Tex && materialTextured(mat, args.tex);
-        vector2 uv(0.0f), dUVdX(0.0f), dUVdY(0.0f);
-        if (textured) {
-            // UV derivatives (resolve.cu:258-275): barycentrics one unit along each
-            // subsample axis from the centroid (for depth of field, along each axis of the
-            // focal-plane offset)
-            float xb0, xb1, xb2, yb0, yb1, yb2;
-            if constexpr (DoF) {
-                dofUVW(T, cam, dofTile, lcfc, lx, ly, dx + 1.0f, dy, xb0, xb1, xb2);
-                dofUVW(T, cam, dofTile, lcfc, lx, ly, dx, dy + 1.0f, yb0, yb1, yb2);
-            } else {
-                pinholeUVW(T, cam, ndir, ndu, ndv, cx + 1.0f, cy, xb0, xb1, xb2);
-                pinholeUVW(T, cam, ndir, ndu, ndv, cx, cy + 1.0f, yb0, yb1, yb2);
-            }
-            uv = V0.uv * bx + V1.uv * by + V2.uv * bz;
-            dUVdX = (V0.uv * xb0 + V1.uv * xb1 + V2.uv * xb2) - uv;
-            dUVdY = (V0.uv * yb0 + V1.uv * yb1 + V2.uv * yb2) - uv;
+        __syncthreads();
+        const uint32_t n = itemCount;
+        for (uint32_t i = tid; i < n; i += Threads) {
+            const uint32_t item = items[i], slot = item / TILE_SIZE, of = item % TILE_SIZE;
+            const GBufferSubsample g = tileBase[(of >> 6) * 64 * A + slot * 64 + (of & 63u)];
+            const ResolveRays r =
+                resolveRays<A, DoF>(args, rot, args.beams[tile * TILE_SIZE + of], tile, of);
+            const vector3 c = shadeSlot<DoF, Half, Tex>(args, cam, dofTile, r, g);
+            colours[item] = c.x;
+            colours[A * TILE_SIZE + item] = c.y;
+            colours[2 * A * TILE_SIZE + item] = c.z;
         }
-        vector3 c;
-        if (textured) {
-            const SurfaceInputs in = surfaceInputs(mat, args.tex, uv, dUVdX, dUVdY);
-            c = Half ? ggxShadeHalf(in, pos, nrm, cam, args.env) : ggxShade(in, pos, nrm, cam, args.env);
-        } else {
-            const MaterialInputs in{mat};
-            c = Half ? ggxShadeHalf(in, pos, nrm, cam, args.env) : ggxShade(in, pos, nrm, cam, args.env);
+        __syncthreads();
+        if (!owner)
+            return;
+#pragma unroll
+        for (int slot = 0; slot < A; slot++) {
+            if (slot >= slots)
+                break;
+            const uint32_t item = uint32_t(slot) * TILE_SIZE + inTile;
+            const vector3 c(colours[item], colours[A * TILE_SIZE + item], colours[2 * A * TILE_SIZE + item]);
+            result += c * float(weight[slot]);
         }
-        result += c * float(__popc(mask));
+    } else {
+        const ResolveRays r = resolveRays<A, DoF>(args, rot, beam, tile, inTile);
+        for (int slot = 0; slot < A; slot++) {
+            GBufferSubsample g;
+            if (!nextSlot(slot, g))
+                break;
+            result += shadeSlot<DoF, Half, Tex>(args, cam, dofTile, r, g) * float(__popc(g.sampleMask));
+        }
     }
     result = result * (1.0f / float(A));
     float r = linearToSRgbFast(acesFilm(result.x));
@@ -398,15 +505,16 @@ __device__ inline void resolveBody(const ResolveArgs& args, uint32_t tile) {
         // hit point of subsample 0 from its barycentrics, projected on the view axis
         float t = INFINITY;
         if (tri0 != badTriIndex) {
+            const ResolveRays rays = resolveRays<A, DoF>(args, rot, beam, tile, inTile);
             PrecomputedTriangleIntersect T = args.tris[tri0];
             float bx, by, bz;
             const vector2 a0 = args.offsets[0];
             if constexpr (DoF) {
-                const vector2 lensUV = args.lensTable[lensBase];
+                const vector2 lensUV = args.lensTable[rays.lensBase];
                 const vector2 dirUV = dofDirUV(a0, dofTile.focalToLensScale, lensUV);
-                dofUVW(T, cam, dofTile, lcfc, lensUV.x, lensUV.y, dirUV.x, dirUV.y, bx, by, bz);
+                dofUVW(T, cam, dofTile, rays.lcfc, lensUV.x, lensUV.y, dirUV.x, dirUV.y, bx, by, bz);
             } else {
-                pinholeUVW(T, cam, ndir, ndu, ndv, a0.x, a0.y, bx, by, bz);
+                pinholeUVW(T, cam, rays.ndir, rays.ndu, rays.ndv, a0.x, a0.y, bx, by, bz);
             }
             const vector3 v1 = T.v0 + T.edge0, v2 = T.v0 + T.edge1;
             const vector3 pos = T.v0 * bx + v1 * by + v2 * bz;
@@ -417,16 +525,16 @@ __device__ inline void resolveBody(const ResolveArgs& args, uint32_t tile) {
 }
 
 template <int A, bool DoF, bool Half, bool Tex>
-__global__ __launch_bounds__(128) void resolveKernel(ResolveArgs args) {
+__global__ __launch_bounds__(64 * resolveWaves(A)) void resolveKernel(ResolveArgs args) {
     resolveBody<A, DoF, Half, Tex>(args, blockIdx.x);
 }
 
 // every tile of the views whose units `start` lists (pinhole views of one MSAA rate and
 // shading precision)
 template <int A, bool Half, bool Tex>
-__global__ __launch_bounds__(128) void resolveBatchKernel(const ResolveArgs* __restrict__ all,
-                                                          const uint32_t* __restrict__ start, uint32_t n,
-                                                          uint32_t swizzle) {
+__global__ __launch_bounds__(64 * resolveWaves(A)) void resolveBatchKernel(const ResolveArgs* __restrict__ all,
+                                                                           const uint32_t* __restrict__ start,
+                                                                           uint32_t n, uint32_t swizzle) {
     const uint32_t unit = xcdUnit(blockIdx.x, gridDim.x, swizzle);
     const uint32_t v = batchView(start, n, unit);
     resolveBody<A, false, Half, Tex>(all[v], unit - start[v]);
@@ -507,16 +615,16 @@ RemapArgs remapArgs(const hvvr_gpu_view* v) {
 
 void launchResolve(hvvr_gpu_view* v, const hvvr_gpu_scene* s, const matrix4x4& m, hipStream_t stream) {
     const ResolveArgs a = resolveArgs(v, s, m);
-    dim3 grid(v->tileCount), block(128);
+    const dim3 grid(v->tileCount);
     const bool dof = v->dof;
     const bool half = v->halfShading;
     const bool tex = s->textureCount > 0;
     switch (v->msaaRate) {
 #define HVVR_RESOLVE_TEX(A, D, F)                                                     \
     if (tex)                                                                          \
-        resolveKernel<A, D, F, true><<<grid, block, 0, stream>>>(a);                  \
+        resolveKernel<A, D, F, true><<<grid, 64 * resolveWaves(A), 0, stream>>>(a);      \
     else                                                                              \
-        resolveKernel<A, D, F, false><<<grid, block, 0, stream>>>(a);
+        resolveKernel<A, D, F, false><<<grid, 64 * resolveWaves(A), 0, stream>>>(a);
 #define HVVR_RESOLVE_CASE(A)                                                          \
     case A:                                                                           \
         if (dof && half) {                                                            \
@@ -551,7 +659,7 @@ void launchResolveBatch(int msaaRate, bool half, bool tex, const ResolveArgs* al
                         uint32_t viewCount, uint32_t units, const LaunchShape& shape, hipStream_t stream) {
     switch (msaaRate) {
 #define HVVR_RESOLVE_BATCH_KERNEL(A, F, T) \
-    resolveBatchKernel<A, F, T><<<units, 128, 0, stream>>>(all, start, viewCount, shape.xcdSwizzle)
+    resolveBatchKernel<A, F, T><<<units, 64 * resolveWaves(A), 0, stream>>>(all, start, viewCount, shape.xcdSwizzle)
 #define HVVR_RESOLVE_BATCH_CASE(A)                                                                            \
     case A:                                                                                                   \
         if (half && tex)                                                                                      \
