@@ -123,7 +123,7 @@ def roofline(stage_ms, survivors, entries, visits, tested, kernel_ms=None):
     tile_lists: algorithmic bytes = 128 B per BVH node visit + 4 B per list entry written,
     against HBM; the node reads mostly hit L2, so beside it stand the HBM bytes the
     counters measured (`traffic`, its fraction of 8 TB/s) and the L2 hit rate: the kernel
-    is bound by the issue and dependency latency of its stack walk, not by either;
+    is bound by the issue and dependency latency of its breadth-first node tests and its sort, not by either;
     intersect: FP32 VALU flops = N_pair (80 + 16 A) with N_pair the (sample, survivor) pairs
     the kernel tested (the tile-cull survivors less those its occlusion skip left out),
     against the FP32 vector figure. `kernel_ms`: the standard tile-list kernel's own average
@@ -158,7 +158,7 @@ def roofline(stage_ms, survivors, entries, visits, tested, kernel_ms=None):
             "hbm_counter_frac": None if traffic is None else round(traffic / t / PEAK_HBM, 5),
             "l2_hit_pct": pmc.get("l2_hit"), "salu_share": pmc.get("salu_share"),
             "valu_busy_pct": pmc.get("valu_busy"),
-            "note": f"issue- and latency-bound stack walk; algorithmic bytes = 128 B x {int(visits)} node visits + "
+            "note": f"issue- and latency-bound node tests and sort; algorithmic bytes = 128 B x {int(visits)} node visits + "
                     f"4 B x {int(entries)} list entries per launch, mostly L2 hits (l2_hit_pct); the HBM bytes "
                     f"the counters measured are `traffic` (hbm_counter_frac of 8 TB/s)"}
 
